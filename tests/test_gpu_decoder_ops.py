@@ -65,6 +65,36 @@ def _attn_ref(x, B, T, nq, nkv, hd, scale, causal):
 
 
 @pytest.mark.parametrize("form", ["auto", "frag"])
+@pytest.mark.parametrize("climb", [5.0, 12.0, -12.0])
+@pytest.mark.parametrize("causal", [1, 0])
+@pytest.mark.parametrize("hd,nq,nkv", [(64, 2, 2), (128, 4, 2), (128, 3, 1)])
+def test_attention_climbing_scores(causal, hd, nq, nkv, climb, form, monkeypatch):
+    """Scores that climb (or fall) by `climb` powers of two from one 32-key block to the next: the
+    online softmax moves its exponent only past 8, so 5 takes it every second block, 12 every
+    block, -12 never.  Bound: a score's operands are split to 2^-22 each, so at |s| <= 7 blocks x
+    12 ln 2 = 58 a probability is off by 58 x 2^-21 = 2.8e-5 at most."""
+    from crispembed_amd import mq
+    import torch
+    if form == "frag":
+        monkeypatch.setenv("MQ_ATTN_SPLIT", "0")
+    B, T = 2, 203
+    x, ld = _qkv(B, T, nq, nkv, hd, hd + nq + causal)
+    x[:, : (nq + nkv) * hd] *= 0.25
+    block = (np.arange(B * T) % T) // 32
+    x[:, 0:nq * hd:hd] = np.sqrt(hd)
+    x[:, nq * hd:(nq + nkv) * hd:hd] = (climb * np.log(2) * block)[:, None]
+    scale = 1.0 / np.sqrt(hd)
+    xd = dev(x)
+    out = torch.full((B * T, nq * hd), float("nan"), dtype=torch.float32, device="cuda")
+    nws = mq.lib().mq_attention_workspace_bytes(B, T, nkv, hd)
+    ws = torch.full((nws // 4,), float("nan"), dtype=torch.float32, device="cuda")
+    mq.check(mq.lib().mq_attention(ctypes.c_void_p(xd.data_ptr()), ld, ctypes.c_void_p(out.data_ptr()), nq * hd, B, T,
+                                   nq, nkv, hd, scale, causal, ctypes.c_void_p(ws.data_ptr()), nws, stream()))
+    ref = _attn_ref(x, B, T, nq, nkv, hd, scale, causal)
+    assert np.abs(host(out) - ref).max() <= 2.8e-5 * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("form", ["auto", "frag"])
 @pytest.mark.parametrize("causal", [1, 0])
 @pytest.mark.parametrize("hd,nq,nkv", [(64, 4, 2), (128, 2, 1), (128, 16, 8), (64, 3, 3), (128, 6, 2)])
 @pytest.mark.parametrize("B,T", [(1, 1), (2, 37), (2, 200), (1, 300)])
