@@ -35,6 +35,7 @@ MQ_SOURCES = [
     ("mq_api.cpp", ["-x", "hip"]),
     ("mq_host_quant.cpp", ["-x", "hip", "-ffp-contract=off"]),
     ("mq_encoder.hip", []),
+    ("mq_rows.hip", []),
     ("mq_bert.cpp", ["-x", "hip"]),
     ("mq_decoder.hip", []),
     ("mq_decoder_run.cpp", ["-x", "hip"]),

@@ -22,6 +22,7 @@
 #include "../../include/mq_bert.h"
 #include "../../include/mq_ops.h"
 #include "mq_internal.h"
+#include "mq_rows.h"
 #include "mq_runner.h"
 
 namespace mq {
@@ -50,7 +51,7 @@ struct mq_bert {
     mq_bert_hparams hp{};
     DevBuf tok, pos, type, lnw, lnb;
     std::vector<Layer> layers;
-    DevBuf x, qkv, att, y, ff, ws, ws2, aws;
+    DevBuf x, x2, qkv, att, y, ff, ws, ws2, aws;
     int64_t rows_cap = 0;
 };
 
@@ -146,6 +147,39 @@ extern "C" int mq_bert_encode(mq_bert *m, const int32_t *ids, const int32_t *typ
                                      (int)H, hp.n_vocab, hp.n_type, s),
                      "embeddings")))
         return rc;
+    // a few rows of Q8_0: five launches a layer (mq_rows.hip), the products' biases added in their
+    // stores; the residual rows alternate between X and X2
+    if (t == MQ_TYPE_Q8_0 && rows_path_fits(rows, T, H, F, (int)(H / hp.n_head)) && (uintptr_t)X % 16 == 0) {
+        if (!m->x2.ensure(rows * H * f4) || !m->ws2.ensure(mq_workspace_bytes(t, rows, F)))
+            return set_error(MQ_ENOMEM, "activation buffers for %lld rows", (long long)rows);
+        float *X2 = m->x2.f();
+        const int var = mq_q8_0_variant();
+        // the product of layer_norm(y + res) (prev: the norm's parameters), of x, or of quantized rows
+        auto product = [&](const Linear &L, const DevBuf &bias, RowsArgs a, void *q_out) {
+            a.bias = bias.f(), a.eps = eps, a.M = (int)rows, a.variant = var;
+            return hip_rc(launch_rows(L.img.p, L.n, L.k, a, q_out, s), "few-row product");
+        };
+        const Layer *prev = nullptr;
+        for (const Layer &L : m->layers) {
+            RowsArgs in, o, up, down;
+            if (prev) in.x = m->y.f(), in.res = X2, in.lw = prev->ln2w.f(), in.lb = prev->ln2b.f(), in.xout = X;
+            else in.x = X;
+            in.y = m->qkv.f();
+            o.x_ws = m->ws.p, o.y = m->y.f();
+            up.x = m->y.f(), up.res = X, up.lw = L.ln1w.f(), up.lb = L.ln1b.f(), up.xout = X2;
+            down.x_ws = m->ws2.p, down.y = m->y.f();
+            if ((rc = product(L.qkv, L.bqkv, in, nullptr)) ||
+                (rc = hip_rc(launch_rows_attn(m->qkv.f(), m->ws.p, var, B, T, (int)H, hp.n_head, s), "attention")) ||
+                (rc = product(L.o, L.bo, o, nullptr)) || (rc = product(L.fc1, L.b1, up, m->ws2.p)) ||
+                (rc = product(L.fc2, L.b2, down, nullptr)))
+                return rc;
+            prev = &L;
+        }
+        if ((rc = hip_rc(launch_bias_res_ln(m->y.f(), nullptr, X2, prev->ln2w.f(), prev->ln2b.f(), eps, X, rows, (int)H, s),
+                         "ffn residual")))
+            return rc;
+        return hip_rc(launch_mean_pool_l2(X, out, B, T, (int)H, s), "pooling");
+    }
     auto mm = [&](const Linear &L, const float *in, float *y) {
         return mq_mul_mat(t, L.img.p, L.n, L.k, in, L.k, rows, y, L.n, m->ws.p, m->ws.bytes, s);
     };

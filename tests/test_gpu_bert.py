@@ -79,3 +79,23 @@ def test_kv_direct_equals_kv_pass(monkeypatch):
     monkeypatch.setenv("MQ_BERT_KV_PASS", "1")
     b = _run(hp, O.Q8_0, 8, 64, "kvd")
     assert np.array_equal(a[2], b[2]) and np.array_equal(a[3], b[3])
+
+
+@pytest.mark.parametrize("H,nh,F,B,T", [
+    (384, 12, 1536, 1, 1), (384, 12, 1536, 1, 31), (384, 12, 1536, 1, 33), (384, 12, 1536, 8, 32), (128, 4, 160, 3, 11),
+    (512, 8, 512, 2, 64), (768, 12, 3072, 1, 64), (1024, 8, 4096, 5, 7), (96, 3, 544, 1, 16)])
+@pytest.mark.parametrize("variant", [0, 2])
+def test_few_rows(oracle, H, nh, F, B, T, variant):
+    """The Q8_0 runner's few-row layers: edges of the 32-row tiles and of the 64-key attention,
+    head_dim 32 / 64 / 128, rows of every register width, widths that are no multiple of 128, two
+    rounding variants of the quantizer (0: x86; 2: reference), against the CPU encoder."""
+    from crispembed_amd import mq
+    hp = dict(SMALL)
+    hp.update(n_embd=H, n_head=nh, n_ff=F, n_max_pos=128)
+    L = mq.lib()
+    saved = L.mq_q8_0_variant()
+    mq.check(L.mq_set_q8_0_variant(variant))
+    try:
+        _check(hp, O.Q8_0, B, T, f"rows_{H}_{F}", oracle)
+    finally:
+        mq.check(L.mq_set_q8_0_variant(saved))
