@@ -14,6 +14,7 @@
 //   GGUF blocks are only 2-byte aligned).
 //   F16 uses v_dot2_f32_f16 on fp16 activations.
 #include "mq_internal.h"
+#include "mq_q8k.h"
 
 #include <climits>
 
@@ -294,8 +295,8 @@ struct GvX {
 // One 256-value superblock sb of rows 0..M-1 of the activation quantized to Q8_K
 // (quantize_row_q8_K: the first value of largest magnitude sets iscale = -127 / max,
 // q = min(127, nearest_int(iscale x)), d = 1 / iscale, the 16-value sums) by one wave: VPL
-// values per lane, 256 / VPL lanes per row, 64 VPL / 256 rows per pass (VPL 4: one row at a
-// time over all 64 lanes; 16: four rows), into this wave's LDS slot laid out as one superblock
+// values per lane, 256 / VPL lanes per row, 64 VPL / 256 rows per pass (VPL 8: two rows at a
+// time; 16: four), into this wave's LDS slot laid out as one superblock
 // of the GEMV activation layout: quants qs[row][256], d ds[row], and the Q4_K min-term operand
 // gs[row][16] (B_j & 63, then 64 (B_j >> 6), B_j the sum of the 32 quants of sub-block j).  The
 // arithmetic is the activation quantizer's (no contraction), so the bytes are the ones it writes.
@@ -373,12 +374,46 @@ __device__ __forceinline__ void gv_quantize_sb(const GvX &X, int sb, int M, int 
     }
 }
 
-// gv_quantize_sb with the lane mapping that keeps the most lanes busy for M rows
-__device__ __forceinline__ void gv_quantize_rows(const GvX &X, int sb, int M, int lane, int8_t *qs, float *ds,
-                                                 _Float16 *gs) {
-    if (M == 1) gv_quantize_sb<4>(X, sb, M, lane, qs, ds, gs);
-    else if (M == 2) gv_quantize_sb<8>(X, sb, M, lane, qs, ds, gs);
-    else gv_quantize_sb<16>(X, sb, M, lane, qs, ds, gs);
+// The one row of a decode step (M = 1): this wave's superblocks sb0, sb0 + 8, ... (NS of them)
+// quantized side by side, lane l holding values 4l .. 4l + 3 of each: every load is in flight
+// before the first is used, the reductions interleave and share the divisions, and the bytes are
+// gv_quantize_sb's.  A decode step is a chain of such kernels, so their latency is its time: with the
+// superblocks one after the other the Q4_K 2048 x 6144 product on silu(gate) up took 9.4 us a
+// launch and a step of 28 layers 708 us, side by side 666 us (MI355X).  At M >= 2 the four-rows-at-once
+// form of gv_quantize_sb is the faster one (a step at M = 2 - 8: 623 against 714 us).
+template <int NS>
+__device__ __forceinline__ void gv_quantize_row(const GvX &X, int sb0, int nsb, int lane, int8_t (*qs)[GEMV_CHUNK * QK_K],
+                                                float (*ds)[GEMV_CHUNK], _Float16 (*gs)[GEMV_CHUNK * 16]) {
+#pragma clang fp contract(off)
+    float4 v[NS], u[NS];
+    const bool silu = X.pre == MQ_PRE_SILU_MUL;
+#pragma unroll
+    for (int i = 0; i < NS; i++) {  // past the end: the last superblock again, not stored
+        const int col = min(sb0 + 8 * i, nsb - 1) * QK_K + 4 * lane;
+        v[i] = *(const float4 *)(X.x + col);
+        if (silu) u[i] = *(const float4 *)(X.x2 + col);
+    }
+    if (silu)
+#pragma unroll
+        for (int i = 0; i < NS; i++) {
+            float4 &g = v[i];
+            g.x = (g.x / (1.0f + expf(-g.x))) * u[i].x, g.y = (g.y / (1.0f + expf(-g.y))) * u[i].y;
+            g.z = (g.z / (1.0f + expf(-g.z))) * u[i].z, g.w = (g.w / (1.0f + expf(-g.w))) * u[i].w;
+        }
+    uint32_t q[NS];
+    int bs[NS];
+    float d[NS];
+    q8_K_rows<NS>(v, lane, q, bs, d);
+#pragma unroll
+    for (int i = 0; i < NS; i++) {
+        if (sb0 + 8 * i >= nsb) continue;  // uniform
+        *(uint32_t *)(qs[i] + 4 * lane) = q[i];
+        if (lane == 0) ds[i][0] = d[i];
+        if ((lane & 7) == 0) {
+            gs[i][lane >> 3] = (_Float16)(bs[i] & 63);
+            gs[i][8 + (lane >> 3)] = (_Float16)((bs[i] >> 6) * 64);
+        }
+    }
 }
 
 template <int TYPE, int SBW, int PF, bool FQ = false>
@@ -419,12 +454,20 @@ __global__ __launch_bounds__(512) void k_gemv_kq_stream(const GvGroups G, const 
         // the first tiles' weights do not depend on the activation: in flight while it is quantized
 #pragma unroll
         for (int f = 0; f < PF; f++) load(ring[f], t + f * (int)gridDim.x);
+        if (live[0]) {
+            const int slot = L.wave * SBW;
+            if (M == 1) {
+                gv_quantize_row<SBW>(X, L.wave, nsb, L.lane, aq + slot, ad + slot, ag + slot);
+            } else {
 #pragma unroll
-        for (int i = 0; i < SBW; i++)
-            if (live[i]) {
-                const int slot = L.wave * SBW + i;
-                gv_quantize_rows(X, L.wave + 8 * i, M, L.lane, aq[slot], ad[slot], ag[slot]);
+                for (int i = 0; i < SBW; i++)
+                    if (live[i]) {
+                        const int sb = L.wave + 8 * i, e = slot + i;
+                        if (M == 2) gv_quantize_sb<8>(X, sb, M, L.lane, aq[e], ad[e], ag[e]);
+                        else gv_quantize_sb<16>(X, sb, M, L.lane, aq[e], ad[e], ag[e]);
+                    }
             }
+        }
         // the wave reads back what its own lanes wrote
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
