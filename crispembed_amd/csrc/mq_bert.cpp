@@ -156,7 +156,7 @@ extern "C" int mq_bert_encode(mq_bert *m, const int32_t *ids, const int32_t *typ
         const int var = mq_q8_0_variant();
         // the product of layer_norm(y + res) (prev: the norm's parameters), of x, or of quantized rows
         auto product = [&](const Linear &L, const DevBuf &bias, RowsArgs a, void *q_out) {
-            a.bias = bias.f(), a.eps = eps, a.M = (int)rows, a.variant = var;
+            a.bias = bias.f(), a.eps = eps, a.ldy = L.n, a.M = (int)rows, a.variant = var;
             return hip_rc(launch_rows(L.img.p, L.n, L.k, a, q_out, s), "few-row product");
         };
         const Layer *prev = nullptr;

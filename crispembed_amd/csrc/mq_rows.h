@@ -6,7 +6,7 @@ namespace mq {
 
 constexpr int ROWS_MAX_K = 4096;   // 16 blocks a wave
 constexpr int ROWS_MAX_LN = 1024;  // rows formed in registers, their quants in LDS
-constexpr int ROWS_MAX_T = 64;     // a wave's lanes as the keys of one query
+constexpr int ROWS_MAX_T = 32;     // keys of one query, a lane each
 
 enum { ROWS_F32 = 0, ROWS_LN = 1, ROWS_Q = 2 };
 
@@ -18,8 +18,9 @@ struct RowsArgs {
     const float *res = nullptr, *lw = nullptr, *lb = nullptr;
     float eps = 0.f;
     float *xout = nullptr;
-    const float *bias = nullptr;  // N floats
-    float *y = nullptr;           // M dense rows of N floats (no q_out)
+    const float *bias = nullptr;  // N floats, or NULL
+    float *y = nullptr;           // M rows of N floats, ldy apart (no q_out)
+    int64_t ldy = 0;
     int M = 0, variant = 0;
     // filled by launch_rows
     const int8_t *wq = nullptr, *xq = nullptr;

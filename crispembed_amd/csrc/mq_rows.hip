@@ -123,29 +123,34 @@ __global__ __launch_bounds__(512) void k_rows(const RowsArgs a) {
 #pragma unroll
             for (int r = 0; r < 4; r++) {
                 if (PRO == ROWS_LN && r < nr) {  // uniform
+                    // the statistics in fp32 (their error scales a whole row, which its blocks' scales
+                    // take up), the values in fp64 up to the one rounding of the result
                     float s = 0.f;
 #pragma unroll
                     for (int p = 0; p < KP; p++) {
-                        float4 &t = v[r][p];
-                        const float4 u = res[PRO == ROWS_LN ? r : 0][p];
-                        t.x += u.x, t.y += u.y, t.z += u.z, t.w += u.w;
-                        s += (t.x + t.y) + (t.z + t.w);
+                        const float4 t = v[r][p], u = res[PRO == ROWS_LN ? r : 0][p];
+                        s += ((t.x + u.x) + (t.y + u.y)) + ((t.z + u.z) + (t.w + u.w));
                     }
                     const float mean = wave_sum_f(s) / (float)a.K;
                     float s2 = 0.f;
 #pragma unroll
                     for (int p = 0; p < KP; p++)
                         if (256 * p + 4 * lane < a.K) {
-                            float4 &t = v[r][p];
-                            t.x -= mean, t.y -= mean, t.z -= mean, t.w -= mean;
-                            s2 += (t.x * t.x + t.y * t.y) + (t.z * t.z + t.w * t.w);
+                            const float4 t = v[r][p], u = res[PRO == ROWS_LN ? r : 0][p];
+                            const float x0 = (t.x + u.x) - mean, x1 = (t.y + u.y) - mean, x2 = (t.z + u.z) - mean,
+                                        x3 = (t.w + u.w) - mean;
+                            s2 += (x0 * x0 + x1 * x1) + (x2 * x2 + x3 * x3);
                         }
-                    const float rstd = 1.0f / sqrtf(wave_sum_f(s2) / (float)a.K + a.eps);
+                    const double rstd = 1.0 / sqrt((double)wave_sum_f(s2) / (double)a.K + (double)a.eps);
 #pragma unroll
                     for (int p = 0; p < KP; p++) {
                         float4 &t = v[r][p];
-                        t.x = t.x * rstd * lw[p].x + lb[p].x, t.y = t.y * rstd * lw[p].y + lb[p].y;
-                        t.z = t.z * rstd * lw[p].z + lb[p].z, t.w = t.w * rstd * lw[p].w + lb[p].w;
+                        const float4 u = res[PRO == ROWS_LN ? r : 0][p];
+                        auto norm = [&](float x, float y, float w, float b) {
+                            return (float)(((double)x + (double)y - (double)mean) * rstd * (double)w + (double)b);
+                        };
+                        t.x = norm(t.x, u.x, lw[p].x, lb[p].x), t.y = norm(t.y, u.y, lw[p].y, lb[p].y);
+                        t.z = norm(t.z, u.z, lw[p].z, lb[p].z), t.w = norm(t.w, u.w, lw[p].w, lb[p].w);
                         const int c = 256 * p + 4 * lane;
                         if (blockIdx.x == 0 && c < a.K) *(float4 *)(a.xout + (int64_t)(m0 + wave + 8 * r) * a.K + c) = t;
                     }
@@ -192,7 +197,11 @@ __global__ __launch_bounds__(512) void k_rows(const RowsArgs a) {
         }
     }
 
-    v16f acc = (v16f){};
+    // fp64 sums of exact terms (19-bit dots times products of two fp16 scales): a chain of launches
+    // leaves the vector units idle, and the fewer roundings, the fewer 8-bit values they move
+    double acc[16];
+#pragma unroll
+    for (int r = 0; r < 16; r++) acc[r] = 0.0;
 #pragma unroll
     for (int i = 0; i < KP; i++) {
         if (wave + 8 * i < nblk) {
@@ -200,32 +209,31 @@ __global__ __launch_bounds__(512) void k_rows(const RowsArgs a) {
             // the tile of d_x d_w (exact: fp16 values), a rank-1 product
             const v16f P = __builtin_amdgcn_mfma_f32_32x32x2f32(half ? 0.f : dx[i], half ? 0.f : dw[i], (v16f){}, 0, 0, 0);
 #pragma unroll
-            for (int r = 0; r < 16; r++) acc[r] += (float)I[r] * P[r];
+            for (int r = 0; r < 16; r++) acc[r] = __builtin_fma((double)I[r], (double)P[r], acc[r]);
         }
     }
     if constexpr (PRO != ROWS_Q) __syncthreads();  // the fragments' space takes the partial tiles
-    float *part = (float *)smem;
+    double *part = (double *)smem;
 #pragma unroll
     for (int r = 0; r < 16; r++) part[(wave * 16 + r) * 64 + lane] = acc[r];
     const int col = n0 + l32;
-    const float bias = col < a.N ? a.bias[col] : 0.f;
+    const float bias = a.bias && col < a.N ? a.bias[col] : 0.f;
     __syncthreads();
 #pragma unroll
     for (int u = 0; u < 2; u++) {
         const int r = 2 * wave + u, row = m0 + 8 * (r / 4) + 4 * half + r % 4;
-        float t[8];  // summed in pairs: fewer roundings on the way of each term
+        double s = bias;
 #pragma unroll
-        for (int w = 0; w < 8; w++) t[w] = part[(w * 16 + r) * 64 + lane];
-        const float s = (((t[0] + t[1]) + (t[2] + t[3])) + ((t[4] + t[5]) + (t[6] + t[7]))) + bias;
+        for (int w = 0; w < 8; w++) s += part[(w * 16 + r) * 64 + lane];
         if constexpr (RQ) {
-            rows_store_q8_0(gelu_erf_f32(s), a.qo, a.qd, a.q_kch, a.q_m_pad, row, blockIdx.x, l32, a.variant, row < a.M);
+            rows_store_q8_0((float)(0.5 * s * (1.0 + erf(s * 0.70710678118654752440))), a.qo, a.qd, a.q_kch, a.q_m_pad, row, blockIdx.x, l32, a.variant, row < a.M);
         } else {
-            if (row < a.M && col < a.N) a.y[(int64_t)row * a.N + col] = s;
+            if (row < a.M && col < a.N) a.y[(int64_t)row * a.ldy + col] = (float)s;
         }
     }
 }
 
-// Attention of one (sequence, head) of at most 64 tokens, fp32: q, k, v (bias added) to LDS, then
+// Attention of one (sequence, head) of at most ROWS_MAX_T tokens, fp32: q, k, v (bias added) to LDS, then
 // a wave per query row, lane j key j: score, softmax over the lanes, and lanes as head dims for
 // the weighted sum of V (64 / HD groups of keys side by side at HD < 64, HD / 64 dims a lane
 // above).  The rows leave as the Q8_0 activation of the o product (32 head dims a block).
@@ -297,7 +305,7 @@ __global__ __launch_bounds__(1024) void k_rows_attn(const float *__restrict__ qk
 
 template <int KP, int PRO, bool RQ>
 static hipError_t rows_cfg(const RowsArgs &a, hipStream_t s) {
-    const size_t op = PRO == ROWS_Q ? 0 : (size_t)(a.K / 32) * (1024 + 128), lds = op > 32768 ? op : 32768;
+    const size_t op = PRO == ROWS_Q ? 0 : (size_t)(a.K / 32) * (1024 + 128), lds = op > 65536 ? op : 65536;
     static_assert(ROWS_MAX_LN / 32 * (1024 + 128) <= 64 * 1024, "no raised LDS limit");
     hipLaunchKernelGGL((k_rows<KP, PRO, RQ>), dim3((unsigned)((a.N + 31) / 32), (unsigned)((a.M + 31) / 32)), dim3(512), lds,
                        s, a);
@@ -350,7 +358,7 @@ hipError_t launch_rows_attn(const float *qkv, void *q_out, int variant, int B, i
     const dim3 g((unsigned)(B * nh));
     const size_t lds = (size_t)3 * T * (hd + 4) * sizeof(float);
     const float scale = 1.0f / sqrtf((float)hd);
-    static std::atomic<bool> attr_set[MQ_MAX_DEVICES];
+    static_assert(3 * ROWS_MAX_T * (128 + 4) * 4 + 4096 <= 64 * 1024, "no raised LDS limit");
     switch (hd) {
         case 32:
             hipLaunchKernelGGL((k_rows_attn<32>), g, dim3(1024), lds, s, qkv, qo, qd, kch, o.m_pad, variant, T, H, nh, scale);
@@ -358,12 +366,9 @@ hipError_t launch_rows_attn(const float *qkv, void *q_out, int variant, int B, i
         case 64:
             hipLaunchKernelGGL((k_rows_attn<64>), g, dim3(1024), lds, s, qkv, qo, qd, kch, o.m_pad, variant, T, H, nh, scale);
             break;
-        case 128: {
-            const hipError_t e = dyn_lds_once((const void *)k_rows_attn<128>, 128 * 1024, attr_set);
-            if (e != hipSuccess) return e;
+        case 128:
             hipLaunchKernelGGL((k_rows_attn<128>), g, dim3(1024), lds, s, qkv, qo, qd, kch, o.m_pad, variant, T, H, nh, scale);
             break;
-        }
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
@@ -373,13 +378,13 @@ hipError_t launch_rows_attn(const float *qkv, void *q_out, int variant, int B, i
 // output columns, so it loses once a launch holds several of them per CU, sooner at wide rows; and
 // its attention walks T / 16 query rows a wave.  MI355X, microseconds a call, GEMM path (GEMV
 // path under 33 rows) / few rows, tokens B x T:
-//   H 384, F 1536, 6 layers:  1x16 486 / 157, 1x32 799 / 190, 1x64 248 / 222, 4x32 248 / 201,
-//                             2x64 249 / 239, 8x32 252 / 244, 4x64 254 / 281, 16x32 273 / 310
-//   H 768, F 3072, 3 layers:  1x16 324 / 126, 1x64 182 / 171, 4x32 185 / 214
-//   H 1024, F 4096, 3 layers: 1x16 374 / 147, 1x64 213 / 193, 4x32 216 / 245
+//   H 384, F 1536, 6 layers:  1x16 489 / 175, 1x32 799 / 214, 2x32 240 / 219, 1x64 243 / 248,
+//                             4x32 243 / 222, 2x64 245 / 252, 16x16 277 / 270, 8x32 247 / 282
+//   H 768, F 3072, 3 layers:  1x16 324 / 138, 2x32 181 / 175, 1x64 181 / 191, 4x32 184 / 248
+//   H 1024, F 4096, 3 layers: 1x16 374 / 165, 2x32 214 / 204, 1x64 211 / 217, 4x32 216 / 283
 // MQ_BERT_ROWS sets the most rows it takes (0: none; measurements).
 bool rows_path_fits(int64_t rows, int64_t T, int64_t H, int64_t F, int hd) {
-    int64_t lim = H > 512 ? 64 : T > 32 ? 128 : 256;
+    int64_t lim = H > 512 ? 64 : 128;
     if (const char *e = getenv("MQ_BERT_ROWS"))
         if (*e) lim = atoi(e);
     return rows <= lim && T <= ROWS_MAX_T && H <= ROWS_MAX_LN && F <= ROWS_MAX_K && H % 32 == 0 && F % 32 == 0 &&

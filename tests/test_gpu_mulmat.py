@@ -65,6 +65,30 @@ def test_gemv(oracle, wtype, m, n, k):
     _check(oracle, wtype, w, x, y, k)
 
 
+@pytest.mark.parametrize("wtype", TYPES)
+@pytest.mark.parametrize("m", [9, 31, 32])
+@pytest.mark.parametrize("n,k", [(33, 32), (1000, 1536), (70, 4096), (65, 4064), (40, 2560), (40, 2816)])
+def test_few_rows_whole_call(oracle, wtype, m, n, k):
+    """mq_mul_mat at 9 - 32 rows: Q8_0 by the few-row product (K up to 4096, every block count a wave
+    may hold), K-quants as a GEMM up to K = 2560, the rest as GEMVs; output rows further apart than n,
+    whose gaps stay untouched."""
+    from crispembed_amd import mq
+    import ctypes
+    import torch
+    if wtype in (O.Q4_K, O.Q6_K) and k % 256:
+        pytest.skip("K-quant rows are whole 256-value superblocks")
+    w, x = _mk(oracle, wtype, m, n, k, m + n + k)
+    _, wp = weight_image(wtype, w, n, k)
+    xd = dev(x)
+    y = torch.full((m, n + 7), -7.0, dtype=torch.float32, device="cuda")
+    P = ctypes.c_void_p
+    mq.check(mq.lib().mq_mul_mat(wtype, wp, n, k, P(xd.data_ptr()), k, m, P(y.data_ptr()), n + 7, None, 0,
+                                 P(torch.cuda.current_stream().cuda_stream)))
+    got = host(y)
+    assert (got[:, n:] == -7.0).all()
+    _check(oracle, wtype, w, x, got[:, :n], k)
+
+
 def test_q8_0_k_tail_and_strides(oracle):
     """k not a multiple of the 128-byte stage; row strides ldx > k and ldy > n."""
     from crispembed_amd import mq
