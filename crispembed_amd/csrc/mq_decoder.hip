@@ -730,7 +730,8 @@ __global__ __launch_bounds__(64 * NW, 2) void k_attn_split(const AttnArgs a, int
 
     // bit j: the wave's key block wave + NW j is fully masked (dead) / has an all-zero mask.
     // Rows 16-byte aligned (m_al): lane l reads 8 keys (16 bytes) of row l / 4 and of row
-    // l / 4 + 16, coalesced; else each lane its own row's 16 keys of the block, 2 bytes at a time.
+    // l / 4 + 16, coalesced; else 2 bytes at a time, a half wave the 32 keys of a row (with its own row
+    // a lane, each load touched 32 cache lines).
     uint64_t dead = 0, zero = 0;
     if constexpr (MK == 1) {
         constexpr int CJ = 2;  // blocks classified per pass
@@ -757,13 +758,14 @@ __global__ __launch_bounds__(64 * NW, 2) void k_attn_split(const AttnArgs a, int
                     }
                     if (j0 + jj >= nj) live[jj] = false, nz[jj] = false;
                 } else {
+                    const int key = kb * 32 + l32;
+                    const bool in = j0 + jj < nj && key < Tk;
 #pragma unroll
                     for (int i = 0; i < 16; i++) {
-                        const int key = kb * 32 + 8 * (i / 4) + 4 * half + (i % 4);
-                        const bool in = j0 + jj < nj && key < Tk;
-                        const float m = (float)mrow[min(key, Tk - 1)];
-                        live[jj] |= in && m != -INFINITY;
-                        nz[jj] |= in && m != 0.0f;
+                        const int row = min(q0 + 2 * i + half, Tq - 1);
+                        const uint32_t m = mbase[(int64_t)row * a.m_sq + min(key, Tk - 1)];
+                        live[jj] |= in && m != 0xFC00u;
+                        nz[jj] |= in && (m & 0x7FFFu) != 0u;
                     }
                 }
             }
