@@ -72,28 +72,20 @@ typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef _Float16 v4h __attribute__((ext_vector_type(4)));
 typedef _Float16 v2h __attribute__((ext_vector_type(2)));
 
-// hi + lo split of floats: hi by one explicit conversion (round toward zero), so that the
-// remainder is formed from the very hi value the MFMA will read.  (A plain (_Float16) cast may be
-// emitted as different conversion instructions for the operand and for the remainder; where their
-// roundings disagree the split loses a 2^-11 term.)  lo is rounded to nearest (operands past
-// fp16's range saturate, as hi does), half the error of the toward-zero pair conversion: the
-// attention's error against fp64 went from 6.5e-7 to 3.9e-7 (head_dim 64, 203 keys).  RTZ selects
-// the pair conversion, cheaper by two instructions a value, for the probabilities, which are split
-// in the attention's inner loop.
-template <bool RTZ = false>
+// hi + lo split of two floats with one explicit rounding (round toward zero) for both
+// halves: the remainder is formed from the very hi value the MFMA will read.  (A plain
+// (_Float16) cast may be emitted as different conversion instructions for the operand and
+// for the remainder; where their roundings disagree the split loses a 2^-11 term.)
 __device__ __forceinline__ void split2(float a, float b, v2h &hi, v2h &lo) {
     hi = __builtin_bit_cast(v2h, __builtin_amdgcn_cvt_pkrtz(a, b));
-    const float ra = a - (float)hi[0], rb = b - (float)hi[1];
-    if constexpr (RTZ) lo = __builtin_bit_cast(v2h, __builtin_amdgcn_cvt_pkrtz(ra, rb));
-    else lo = v2h{(_Float16)fminf(fmaxf(ra, -65504.f), 65504.f), (_Float16)fminf(fmaxf(rb, -65504.f), 65504.f)};
+    lo = __builtin_bit_cast(v2h, __builtin_amdgcn_cvt_pkrtz(a - (float)hi[0], b - (float)hi[1]));
 }
 
-template <bool RTZ = false>
 __device__ __forceinline__ void split8(const float (&x)[8], v8h &hi, v8h &lo) {
 #pragma unroll
     for (int j = 0; j < 8; j += 2) {
         v2h h, l;
-        split2<RTZ>(x[j], x[j + 1], h, l);
+        split2(x[j], x[j + 1], h, l);
         hi[j] = h[0], hi[j + 1] = h[1], lo[j] = l[0], lo[j + 1] = l[1];
     }
 }

@@ -65,6 +65,50 @@ def _attn_ref(x, B, T, nq, nkv, hd, scale, causal):
 
 
 @pytest.mark.parametrize("form", ["auto", "frag"])
+@pytest.mark.parametrize("g", [12, 14, 16])
+@pytest.mark.parametrize("causal", [1, 0])
+@pytest.mark.parametrize("hd,nq,nkv", [(64, 2, 2), (128, 4, 2)])
+def test_attention_sink(causal, hd, nq, nkv, g, form, monkeypatch):
+    """An attention sink: key 0 stands g to g + 1 octaves above every other key and its value is 0, so
+    the output comes from the small probabilities alone.  Scores and values are exact in fp16 (and
+    in fp32 after the base-2 scaling), which leaves the 2^x (2 ulp), the fp32 sums and division (2^-21
+    together) and the split of P: 22 bits, and 2^-39 of the row's largest probability below 2^-17 of
+    it, i.e. 2^(g + 1 - 39) of a small one."""
+    from crispembed_amd import mq
+    import torch
+    if form == "frag":
+        monkeypatch.setenv("MQ_ATTN_SPLIT", "0")
+    B, T = 2, 512
+    rng = np.random.default_rng(hd + g)
+    scale = 1.0 / np.sqrt(hd)
+    qscale = np.float32(np.float32(scale) * np.float32(1.4426950408889634))  # score octaves per unit of q . k
+    q0 = np.float32(1.0) / qscale
+    q0 = next(c for c in (q0, np.nextafter(q0, np.float32(0)), np.nextafter(q0, np.float32(99)))
+              if np.float32(c * qscale) == np.float32(1.0))
+    x = np.zeros((B, T, nq + 2 * nkv, hd), np.float32)
+    x[:, :, :nq, 0] = q0
+    octaves = rng.integers(0, 1024, (B, T, nkv)) / -1024.0  # the small keys' scores, in (-1, 0]
+    octaves[:, 0] = g
+    x[:, :, nq:nq + nkv, 0] = octaves
+    x[:, 1:, nq + nkv:] = rng.standard_normal((B, T - 1, nkv, hd)).astype(np.float16)
+    v = x[:, :, nq + nkv:].astype(np.float64)
+    p = np.exp2(octaves - g)
+    if causal:
+        o = np.cumsum(p[..., None] * v, 1) / np.cumsum(p, 1)[..., None]
+    else:
+        o = np.broadcast_to(((p[..., None] * v).sum(1) / p.sum(1)[..., None])[:, None], v.shape)
+    ref = np.repeat(o, nq // nkv, axis=2).reshape(B * T, nq * hd)
+    ld = (nq + 2 * nkv) * hd
+    xd = dev(x.reshape(B * T, ld))
+    out = torch.full((B * T, nq * hd), float("nan"), dtype=torch.float32, device="cuda")
+    nws = mq.lib().mq_attention_workspace_bytes(B, T, nkv, hd)
+    ws = torch.full((nws // 4,), float("nan"), dtype=torch.float32, device="cuda")
+    mq.check(mq.lib().mq_attention(ctypes.c_void_p(xd.data_ptr()), ld, ctypes.c_void_p(out.data_ptr()), nq * hd, B, T,
+                                   nq, nkv, hd, scale, causal, ctypes.c_void_p(ws.data_ptr()), nws, stream()))
+    assert np.linalg.norm(host(out) - ref) <= (2.0 ** -21 + 2.0 ** (g - 38)) * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("form", ["auto", "frag"])
 @pytest.mark.parametrize("climb", [5.0, 12.0, -12.0])
 @pytest.mark.parametrize("causal", [1, 0])
 @pytest.mark.parametrize("hd,nq,nkv", [(64, 2, 2), (128, 4, 2), (128, 3, 1)])
