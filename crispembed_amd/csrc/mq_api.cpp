@@ -311,31 +311,25 @@ int mq_mul_mat_path(int type, int64_t n, int64_t k, int64_t m) {
     return MQ_PATH_GEMM;
 }
 
-// What a whole mq_mul_mat makes of the 9 - 32 row products that mq_mul_mat_path leaves to the GEMV (a
-// caller that quantizes and multiplies in two calls keeps that layout): two launches whatever m is,
-// where the GEMV takes a quantizer and a pass over the weights per 8 rows.  K-quants run as a GEMM
-// up to K = 2560 (past that its few workgroups walk K alone for longer, and its one chain of
-// sums rounds more than the GEMV's eight), Q8_0 as the encoder's few-row product, whose eight waves
-// split K; F16 stays (the GEMM's sums round twice as much).  MI355X, microseconds a call, GEMV / here,
-// at m = 9, 16, 24, 32:
-//   Q4_K 1024 x 1024  15 / 10, 15 / 10, 21 / 10, 26 / 10    (1024 x 4096  15 / 22, 15 / 23, 23 / 23, 31 / 23)
-//   Q6_K 6144 x 2048  16 / 12, 17 / 14, 27 / 12, 35 / 12    (1024 x 4096  16 / 18, 18 / 18, 27 / 19, 36 / 19)
-enum { FEW_GEMV, FEW_GEMM, FEW_ROWS };
-static int few_rows_form(int type, int64_t n, int64_t k, int64_t m) {
-    if (m <= GEMV_CHUNK || mq_mul_mat_path(type, n, k, m) != MQ_PATH_GEMV) return FEW_GEMV;
-    if (type == MQ_TYPE_Q8_0) return k <= ROWS_MAX_K ? FEW_ROWS : FEW_GEMV;
-    return (type == MQ_TYPE_Q4_K || type == MQ_TYPE_Q6_K) && k <= 2560 ? FEW_GEMM : FEW_GEMV;
+// Of the 9 - 32 row products that mq_mul_mat_path leaves to the GEMV, a whole mq_mul_mat (a caller
+// that quantizes and multiplies in two calls keeps that layout) takes Q8_0 as the encoder's few-row
+// product: two launches whatever m is, where the GEMV takes a quantizer and a pass over the weights
+// per 8 rows.  The K-quants and F16 stay: their GEMM is faster at some of these sizes (Q4_K 1024 x 1024
+// at 32 rows 26 -> 10 us) and slower at others (1024 x 4096 at 9 rows 15 -> 22 us), and its one chain
+// of sums rounds more than the GEMV's eight.
+static bool few_rows(int type, int64_t n, int64_t k, int64_t m) {
+    return type == MQ_TYPE_Q8_0 && m > GEMV_CHUNK && k <= ROWS_MAX_K && mq_mul_mat_path(type, n, k, m) == MQ_PATH_GEMV;
 }
 
 // the quantizer and the product of a whole mq_mul_mat, ws large enough for either layout
 static int quantize_and_multiply(int type, const void *w_image, int64_t n, int64_t k, const float *x, int64_t ldx,
                                  int64_t m, float *y, int64_t ldy, void *ws, size_t ws_bytes, int path, bool choose,
                                  void *stream) {
-    const int few = choose ? few_rows_form(type, n, k, m) : FEW_GEMV;
-    if (few != FEW_GEMV) path = MQ_PATH_GEMM;
+    const bool few = choose && few_rows(type, n, k, m);
+    if (few) path = MQ_PATH_GEMM;
     const int rc = mq_quantize_act(type, x, ldx, m, k, ws, ws_bytes, path, stream);
     if (rc) return rc;
-    if (few == FEW_ROWS) {
+    if (few) {
         RowsArgs a;
         a.x_ws = ws, a.y = y, a.ldy = ldy, a.M = (int)m, a.variant = mq_q8_0_variant();
         const hipError_t e = launch_rows(w_image, n, k, a, nullptr, (hipStream_t)stream);

@@ -70,8 +70,7 @@ def test_gemv(oracle, wtype, m, n, k):
 @pytest.mark.parametrize("n,k", [(33, 32), (1000, 1536), (70, 4096), (65, 4064), (40, 2560), (40, 2816)])
 def test_few_rows_whole_call(oracle, wtype, m, n, k):
     """mq_mul_mat at 9 - 32 rows: Q8_0 by the few-row product (K up to 4096, every block count a wave
-    may hold), K-quants as a GEMM up to K = 2560, the rest as GEMVs; output rows further apart than n,
-    whose gaps stay untouched."""
+    may hold), the rest as GEMVs; output rows further apart than n, whose gaps stay untouched."""
     from crispembed_amd import mq
     import ctypes
     import torch
@@ -87,6 +86,22 @@ def test_few_rows_whole_call(oracle, wtype, m, n, k):
     got = host(y)
     assert (got[:, n:] == -7.0).all()
     _check(oracle, wtype, w, x, got[:, :n], k)
+
+
+@pytest.mark.parametrize("wtype", [O.Q4_K, O.Q6_K, O.F16])
+@pytest.mark.parametrize("m", [8, 9, 17, 32, 33])
+@pytest.mark.parametrize("n,k", [(1000, 256), (33, 2048), (40, 2560), (65, 2816)])
+def test_whole_call_equals_the_reported_path(oracle, wtype, m, n, k):
+    """mq_mul_mat gives what quantizing and multiplying on the path that mq_mul_mat_path names gives, bit
+    for bit: a whole call may take fewer launches, but its sums round no differently."""
+    from crispembed_amd import mq
+    L = mq.lib()
+    w, x = _mk(oracle, wtype, m, n, k, 3 * m + n + k)
+    _, wp = weight_image(wtype, w, n, k)
+    xd = dev(x)
+    whole = host(mul_mat(wtype, wp, n, k, xd))
+    path = L.mq_mul_mat_path(wtype, n, k, m)
+    assert np.array_equal(whole, host(mul_mat(wtype, wp, n, k, xd, path=path)))
 
 
 def test_q8_0_k_tail_and_strides(oracle):
