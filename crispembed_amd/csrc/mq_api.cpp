@@ -314,7 +314,7 @@ int mq_mul_mat_path(int type, int64_t n, int64_t k, int64_t m) {
 // Of the 9 - 32 row products that mq_mul_mat_path leaves to the GEMV, a whole mq_mul_mat (a caller
 // that quantizes and multiplies in two calls keeps that layout) takes Q8_0 as the encoder's few-row
 // product: two launches whatever m is, where the GEMV takes a quantizer and a pass over the weights
-// per 8 rows.  The K-quants and F16 stay: their GEMM is faster at some of these sizes (Q4_K 1024 x 1024
+// per 8 rows, and the GEMV's sums bit for bit.  The K-quants and F16 stay: their GEMM is faster at some of these sizes (Q4_K 1024 x 1024
 // at 32 rows 26 -> 10 us) and slower at others (1024 x 4096 at 9 rows 15 -> 22 us), and its one chain
 // of sums rounds more than the GEMV's eight.
 static bool few_rows(int type, int64_t n, int64_t k, int64_t m) {

@@ -31,8 +31,9 @@ struct RowsArgs {
     int n_pad = 0, kch = 0, q_kch = 0, N = 0, K = 0;
 };
 
-// y = rows w^T + bias for a prepared Q8_0 weight image of n x k; with q_out instead gelu_erf of
-// that, as the Q8_0 activation of the next product (the GEMM workspace layout of M rows of n)
+// y = rows w^T + bias for a prepared Q8_0 weight image of n x k, with the GEMV's sums bit for bit;
+// with q_out (LayerNorm prologue only) instead gelu_erf of that, as the Q8_0 activation of the next
+// product (the GEMM workspace layout of M rows of n)
 hipError_t launch_rows(const void *image, int64_t n, int64_t k, RowsArgs a, void *q_out, hipStream_t s);
 // full attention over q|k|v rows of 3 H floats (bias added), T at most ROWS_MAX_T; the rows leave
 // as the Q8_0 activation of the o product in q_out

@@ -13,6 +13,7 @@
 // workgroup can quantize for the next kernel (its 32 columns are one Q8_0 block of each row) it
 // does in its store.
 #include <cstdlib>
+#include <type_traits>
 
 #include "mq_internal.h"
 #include "mq_act.h"
@@ -57,8 +58,25 @@ __device__ __forceinline__ void rows_store_q8_0(float x, int8_t *qo, float *qd, 
     }
 }
 
-// 8 waves; wave w multiplies the 32-value blocks w, w + 8, ... of K (one v_mfma_i32_32x32x32_i8
-// and a scaled add each, as the GEMM), and the eight partial tiles meet in LDS.
+// The few-row product.  8 waves; wave w multiplies the 32-value blocks w, w + 8, ... of K (one
+// v_mfma_i32_32x32x32_i8 and a scaled add each), and the eight partial tiles meet in LDS.  The sums
+// are the GEMV's, in its order, so the results are its results bit for bit: there lane l of a wave
+// adds up blocks l and l + 64 and the lanes meet in a tree over lane ^ 32, 16, 8, 4, 2, 1; here block
+// l = w + 8 i is step i of wave w, so the tree's first three levels join steps i ^ 4, 2, 1 of a wave
+// and the last three join waves w ^ 4, 2, 1.
+// rows_tree<KP, I, S>: the sum of steps I, I + S, I + 2 S, ... < min(KP, 8), as the GEMV's lanes meet
+// (a step that is not there is +0 in the GEMV, and no step's sum is -0: it drops out)
+template <int KP, int I, int S, class F>
+__device__ __forceinline__ v16f rows_tree(F &&leaf) {
+    if constexpr (S == 8) {
+        return leaf(std::integral_constant<int, I>{});
+    } else {
+        v16f t = rows_tree<KP, I, 2 * S>(leaf);
+        if constexpr (I + S < (KP < 8 ? KP : 8)) t += rows_tree<KP, I + S, 2 * S>(leaf);
+        return t;
+    }
+}
+
 // PRO: the rows.  ROWS_Q: quantized already (GEMM layout), fragments straight to registers.
 // ROWS_F32, ROWS_LN: wave w forms rows w, w + 8, w + 16, w + 24 (lane l values 256 p + 4 l .. + 3, p < KP =
 // ceil(K / 256)), as they are or as layer_norm(x + res), quantizes them and leaves them in LDS
@@ -197,23 +215,24 @@ __global__ __launch_bounds__(512) void k_rows(const RowsArgs a) {
         }
     }
 
-    // fp64 sums of exact terms (19-bit dots times products of two fp16 scales): a chain of launches
-    // leaves the vector units idle, and the fewer roundings, the fewer 8-bit values they move
-    double acc[16];
+    // steps i and i + 8: the exact dot times the exact product of the two fp16 scales
+    auto leaf = [&](auto ic) __attribute__((always_inline)) {
+        constexpr int i = decltype(ic)::value;
+        v16f t = (v16f){};
 #pragma unroll
-    for (int r = 0; r < 16; r++) acc[r] = 0.0;
+        for (int u = i; u < KP; u += 8)
+            if (wave + 8 * u < nblk) {  // uniform
+                const v16i I = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[u], wf[u], (v16i){}, 0, 0, 0);
+                // the tile of d_x d_w, a rank-1 product
+                const v16f P = __builtin_amdgcn_mfma_f32_32x32x2f32(half ? 0.f : dx[u], half ? 0.f : dw[u], (v16f){}, 0, 0, 0);
 #pragma unroll
-    for (int i = 0; i < KP; i++) {
-        if (wave + 8 * i < nblk) {
-            const v16i I = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[i], wf[i], (v16i){}, 0, 0, 0);
-            // the tile of d_x d_w (exact: fp16 values), a rank-1 product
-            const v16f P = __builtin_amdgcn_mfma_f32_32x32x2f32(half ? 0.f : dx[i], half ? 0.f : dw[i], (v16f){}, 0, 0, 0);
-#pragma unroll
-            for (int r = 0; r < 16; r++) acc[r] = __builtin_fma((double)I[r], (double)P[r], acc[r]);
-        }
-    }
+                for (int r = 0; r < 16; r++) t[r] = __builtin_fmaf((float)I[r], P[r], t[r]);
+            }
+        return t;
+    };
+    const v16f acc = rows_tree<KP, 0, 1>(leaf);
     if constexpr (PRO != ROWS_Q) __syncthreads();  // the fragments' space takes the partial tiles
-    double *part = (double *)smem;
+    float *part = (float *)smem;
 #pragma unroll
     for (int r = 0; r < 16; r++) part[(wave * 16 + r) * 64 + lane] = acc[r];
     const int col = n0 + l32;
@@ -222,13 +241,15 @@ __global__ __launch_bounds__(512) void k_rows(const RowsArgs a) {
 #pragma unroll
     for (int u = 0; u < 2; u++) {
         const int r = 2 * wave + u, row = m0 + 8 * (r / 4) + 4 * half + r % 4;
-        double s = bias;
+        float w[8];
 #pragma unroll
-        for (int w = 0; w < 8; w++) s += part[(w * 16 + r) * 64 + lane];
+        for (int v = 0; v < 8; v++) w[v] = part[(v * 16 + r) * 64 + lane];
+        float s = ((w[0] + w[4]) + (w[2] + w[6])) + ((w[1] + w[5]) + (w[3] + w[7]));
+        if (a.bias) s += bias;
         if constexpr (RQ) {
-            rows_store_q8_0((float)(0.5 * s * (1.0 + erf(s * 0.70710678118654752440))), a.qo, a.qd, a.q_kch, a.q_m_pad, row, blockIdx.x, l32, a.variant, row < a.M);
+            rows_store_q8_0(gelu_erf_f32(s), a.qo, a.qd, a.q_kch, a.q_m_pad, row, blockIdx.x, l32, a.variant, row < a.M);
         } else {
-            if (row < a.M && col < a.N) a.y[(int64_t)row * a.ldy + col] = (float)s;
+            if (row < a.M && col < a.N) a.y[(int64_t)row * a.ldy + col] = s;
         }
     }
 }
@@ -303,18 +324,13 @@ __global__ __launch_bounds__(1024) void k_rows_attn(const float *__restrict__ qk
     }
 }
 
-template <int KP, int PRO, bool RQ>
+template <int KP, int PRO, bool RQ = false>
 static hipError_t rows_cfg(const RowsArgs &a, hipStream_t s) {
-    const size_t op = PRO == ROWS_Q ? 0 : (size_t)(a.K / 32) * (1024 + 128), lds = op > 65536 ? op : 65536;
+    const size_t op = PRO == ROWS_Q ? 0 : (size_t)(a.K / 32) * (1024 + 128), lds = op > 32768 ? op : 32768;
     static_assert(ROWS_MAX_LN / 32 * (1024 + 128) <= 64 * 1024, "no raised LDS limit");
     hipLaunchKernelGGL((k_rows<KP, PRO, RQ>), dim3((unsigned)((a.N + 31) / 32), (unsigned)((a.M + 31) / 32)), dim3(512), lds,
                        s, a);
     return hipGetLastError();
-}
-
-template <int KP, int PRO>
-static hipError_t rows_out(const RowsArgs &a, hipStream_t s) {
-    return a.qo ? rows_cfg<KP, PRO, true>(a, s) : rows_cfg<KP, PRO, false>(a, s);
 }
 
 hipError_t launch_rows(const void *image, int64_t n, int64_t k, RowsArgs a, void *q_out, hipStream_t s) {
@@ -336,16 +352,22 @@ hipError_t launch_rows(const void *image, int64_t n, int64_t k, RowsArgs a, void
         const ActPlanes x = act_planes(MQ_TYPE_Q8_0, a.M, k, true);
         a.xq = (const int8_t *)a.x_ws + x.xq, a.xd = (const float *)((const char *)a.x_ws + x.xd);
         a.m_pad = x.m_pad;
-        if (k <= 512) return rows_out<2, ROWS_Q>(a, s);
-        if (k <= 1024) return rows_out<4, ROWS_Q>(a, s);
-        if (k <= 1536) return rows_out<6, ROWS_Q>(a, s);
-        return rows_out<16, ROWS_Q>(a, s);
+        if (a.qo) return hipErrorInvalidValue;
+        // steps a wave: each one that is not there still costs its (clamped) loads
+        if (k <= 512) return rows_cfg<2, ROWS_Q>(a, s);
+        if (k <= 1024) return rows_cfg<4, ROWS_Q>(a, s);
+        if (k <= 1536) return rows_cfg<6, ROWS_Q>(a, s);
+        if (k <= 2048) return rows_cfg<8, ROWS_Q>(a, s);
+        if (k <= 3072) return rows_cfg<12, ROWS_Q>(a, s);
+        return rows_cfg<16, ROWS_Q>(a, s);
     }
     if (k > ROWS_MAX_LN || (a.res && (!a.xout || a.xout == a.res || a.xout == a.x)) ||
         ((uintptr_t)a.x | (uintptr_t)a.res | (uintptr_t)a.lw | (uintptr_t)a.lb | (uintptr_t)a.xout) % 16)
         return hipErrorInvalidValue;
-    if (a.res) return k <= 512 ? rows_out<2, ROWS_LN>(a, s) : rows_out<4, ROWS_LN>(a, s);
-    return k <= 512 ? rows_out<2, ROWS_F32>(a, s) : rows_out<4, ROWS_F32>(a, s);
+    if (a.res && a.qo) return k <= 512 ? rows_cfg<2, ROWS_LN, true>(a, s) : rows_cfg<4, ROWS_LN, true>(a, s);
+    if (a.res) return k <= 512 ? rows_cfg<2, ROWS_LN>(a, s) : rows_cfg<4, ROWS_LN>(a, s);
+    if (a.qo) return hipErrorInvalidValue;
+    return k <= 512 ? rows_cfg<2, ROWS_F32>(a, s) : rows_cfg<4, ROWS_F32>(a, s);
 }
 
 hipError_t launch_rows_attn(const float *qkv, void *q_out, int variant, int B, int T, int H, int nh, hipStream_t s) {

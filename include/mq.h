@@ -138,7 +138,7 @@ int mq_weight_prepare(int type, void *image, int64_t n, int64_t k, int64_t row0,
 /* The path MQ_PATH_AUTO of mq_mul_mat / mq_mul_mat_ex takes for an n x k weight and m rows:
  * MQ_PATH_GEMV up to mq_gemv_max_m() rows, and up to 32 rows while a 128 x 128 GEMM tile grid
  * would have fewer than 64 workgroups (short inputs on narrow layers); else MQ_PATH_GEMM.
- * (For some of the 9 - 32 row products a whole mq_mul_mat call takes a faster form of its own.)
+ * (A whole mq_mul_mat call of 9 - 32 Q8_0 rows runs the GEMV's sums in fewer launches: same bits.)
  * Callers of the two-step API (mq_quantize_act_ex + mq_mul_mat_q*) pass it to both calls. */
 int mq_mul_mat_path(int type, int64_t n, int64_t k, int64_t m);
 size_t mq_workspace_bytes(int type, int64_t m, int64_t k);

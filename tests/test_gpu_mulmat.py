@@ -88,13 +88,16 @@ def test_few_rows_whole_call(oracle, wtype, m, n, k):
     _check(oracle, wtype, w, x, got[:, :n], k)
 
 
-@pytest.mark.parametrize("wtype", [O.Q4_K, O.Q6_K, O.F16])
+@pytest.mark.parametrize("wtype", TYPES)
 @pytest.mark.parametrize("m", [8, 9, 17, 32, 33])
-@pytest.mark.parametrize("n,k", [(1000, 256), (33, 2048), (40, 2560), (65, 2816)])
+@pytest.mark.parametrize("n,k", [(1000, 256), (33, 2048), (40, 2560), (65, 2816), (96, 32), (70, 1536), (31, 480),
+                                 (40, 992), (129, 3072), (64, 4064), (100, 4096)])
 def test_whole_call_equals_the_reported_path(oracle, wtype, m, n, k):
     """mq_mul_mat gives what quantizing and multiplying on the path that mq_mul_mat_path names gives, bit
     for bit: a whole call may take fewer launches, but its sums round no differently."""
     from crispembed_amd import mq
+    if wtype in (O.Q4_K, O.Q6_K) and k % 256:
+        pytest.skip("K-quant rows are whole 256-value superblocks")
     L = mq.lib()
     w, x = _mk(oracle, wtype, m, n, k, 3 * m + n + k)
     _, wp = weight_image(wtype, w, n, k)
