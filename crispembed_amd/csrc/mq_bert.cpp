@@ -147,18 +147,20 @@ extern "C" int mq_bert_encode(mq_bert *m, const int32_t *ids, const int32_t *typ
                                      (int)H, hp.n_vocab, hp.n_type, s),
                      "embeddings")))
         return rc;
-    // a few rows of Q8_0: five launches a layer (mq_rows.hip), the products' biases added in their
-    // stores; the residual rows alternate between X and X2
+    // a few rows of Q8_0: five launches a layer (mq_rows.hip) with the values of the loop below, bit for
+    // bit; the products' biases added in their stores, the residual rows alternating between X and X2
     if (t == MQ_TYPE_Q8_0 && rows_path_fits(rows, T, H, F, (int)(H / hp.n_head)) && (uintptr_t)X % 16 == 0) {
         if (!m->x2.ensure(rows * H * f4) || !m->ws2.ensure(mq_workspace_bytes(t, rows, F)))
             return set_error(MQ_ENOMEM, "activation buffers for %lld rows", (long long)rows);
         float *X2 = m->x2.f();
         const int var = mq_q8_0_variant();
         // the product of layer_norm(y + res) (prev: the norm's parameters), of x, or of quantized rows
-        auto product = [&](const Linear &L, const DevBuf &bias, RowsArgs a, void *q_out) {
+        auto product = [&](const Linear &L, const DevBuf &bias, RowsArgs a, void *q_out, bool groups = false) {
             a.bias = bias.f(), a.eps = eps, a.ldy = L.n, a.M = (int)rows, a.variant = var;
-            return hip_rc(launch_rows(L.img.p, L.n, L.k, a, q_out, s), "few-row product");
+            return hip_rc(groups ? launch_rows_groups(L.img.p, L.n, L.k, a, s) : launch_rows(L.img.p, L.n, L.k, a, q_out, s),
+                          "few-row product");
         };
+        const bool down_groups = rows > mq_gemv_max_m();  // the FFN-down product is the GEMM's past the GEMV's rows
         const Layer *prev = nullptr;
         for (const Layer &L : m->layers) {
             RowsArgs in, o, up, down;
@@ -171,7 +173,7 @@ extern "C" int mq_bert_encode(mq_bert *m, const int32_t *ids, const int32_t *typ
             if ((rc = product(L.qkv, L.bqkv, in, nullptr)) ||
                 (rc = hip_rc(launch_rows_attn(m->qkv.f(), m->ws.p, var, B, T, (int)H, hp.n_head, s), "attention")) ||
                 (rc = product(L.o, L.bo, o, nullptr)) || (rc = product(L.fc1, L.b1, up, m->ws2.p)) ||
-                (rc = product(L.fc2, L.b2, down, nullptr)))
+                (rc = product(L.fc2, L.b2, down, nullptr, down_groups)))
                 return rc;
             prev = &L;
         }

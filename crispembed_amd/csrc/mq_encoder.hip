@@ -20,25 +20,14 @@ constexpr int LN_MAXV = 16;  // values per lane: rows up to 1024 wide
 // One wave per row: y = (x - mean) / sqrt(var + eps) * w + b, x held in registers
 // (V values per lane, rows up to 64*V wide).
 template <int V>
-__device__ __forceinline__ void ln_row(float (&v)[V], int n, int lane, const float *w, const float *b, float eps,
+__device__ __forceinline__ void ln_row(const float (&v)[V], int n, int lane, const float *w, const float *b, float eps,
                                        float *out) {
-    float s = 0.f;
-#pragma unroll
-    for (int i = 0; i < V; i++)
-        if (lane + 64 * i < n) s += v[i];
-    const float mean = wave_sum_f(s) / (float)n;
-    float s2 = 0.f;
-#pragma unroll
-    for (int i = 0; i < V; i++)
-        if (lane + 64 * i < n) {
-            v[i] -= mean;
-            s2 += v[i] * v[i];
-        }
-    const float rstd = 1.0f / sqrtf(wave_sum_f(s2) / (float)n + eps);
+    float mean, rstd;
+    ln_stats(v, n, lane, eps, mean, rstd);
 #pragma unroll
     for (int i = 0; i < V; i++) {
         const int c = lane + 64 * i;
-        if (c < n) out[c] = v[i] * rstd * w[c] + b[c];
+        if (c < n) out[c] = ln_value(v[i], mean, rstd, w[c], b[c]);
     }
 }
 
@@ -96,7 +85,7 @@ __global__ __launch_bounds__(256) void k_bias_res_ln(const float *__restrict__ y
 // wave read the same K / V row at a time, an LDS broadcast), then the KS partial states of
 // each row are merged through LDS (the K / V space, free by then):
 //   m = max m_s,  l = sum l_s e^(m_s - m),  o = sum o_s e^(m_s - m) / l.
-constexpr int ATT_KB = 16;
+
 template <int HD, int KS>
 __global__ __launch_bounds__(512) void k_attention(const float *__restrict__ qkv, const float *__restrict__ bqkv,
                                                    float *__restrict__ out, int T, int H, int nh, float scale) {
@@ -138,10 +127,8 @@ __global__ __launch_bounds__(512) void k_attention(const float *__restrict__ qkv
                 const float4 *kr = (const float4 *)(Ks + (j0 + jj) * HD);
                 float sv = 0.f;
 #pragma unroll
-                for (int d4 = 0; d4 < HD / 4; d4++) {
-                    const float4 kv = kr[d4];
-                    sv += q[4 * d4] * kv.x + q[4 * d4 + 1] * kv.y + q[4 * d4 + 2] * kv.z + q[4 * d4 + 3] * kv.w;
-                }
+                for (int d4 = 0; d4 < HD / 4; d4++)
+                    sv = score4(sv, make_float4(q[4 * d4], q[4 * d4 + 1], q[4 * d4 + 2], q[4 * d4 + 3]), kr[d4]);
                 sc[jj] = sv;
                 bm = fmaxf(bm, sv);
             }
@@ -161,10 +148,10 @@ __global__ __launch_bounds__(512) void k_attention(const float *__restrict__ qkv
 #pragma unroll
                 for (int d4 = 0; d4 < HD / 4; d4++) {
                     const float4 vv = vr[d4];
-                    o[4 * d4] += p * vv.x;
-                    o[4 * d4 + 1] += p * vv.y;
-                    o[4 * d4 + 2] += p * vv.z;
-                    o[4 * d4 + 3] += p * vv.w;
+                    o[4 * d4] = __builtin_fmaf(p, vv.x, o[4 * d4]);
+                    o[4 * d4 + 1] = __builtin_fmaf(p, vv.y, o[4 * d4 + 1]);
+                    o[4 * d4 + 2] = __builtin_fmaf(p, vv.z, o[4 * d4 + 2]);
+                    o[4 * d4 + 3] = __builtin_fmaf(p, vv.w, o[4 * d4 + 3]);
                 }
             }
         }
@@ -189,16 +176,17 @@ __global__ __launch_bounds__(512) void k_attention(const float *__restrict__ qkv
             float m = mx;
 #pragma unroll
             for (int k = 1; k < KS; k++) m = fmaxf(m, sm[(int64_t)((k - 1) * T + i) * (HD + 2)]);
-            float w0 = expf(mx - m), lt = l * w0;
-#pragma unroll
-            for (int d = 0; d < HD; d++) o[d] *= w0;
+            const float w0 = expf(mx - m);
+            float lt = l;
 #pragma unroll
             for (int k = 1; k < KS; k++) {
                 const float *sk = sm + (int64_t)((k - 1) * T + i) * (HD + 2);
                 const float w = expf(sk[0] - m);
-                lt += sk[1] * w;
+                // k = 1: the other range's product rounds on its own, this one's with the sum
+                lt = k == 1 ? __builtin_fmaf(lt, w0, sk[1] * w) : __builtin_fmaf(sk[1], w, lt);
 #pragma unroll
-                for (int d = 0; d < HD; d++) o[d] += sk[2 + d] * w;
+                for (int d = 0; d < HD; d++)
+                    o[d] = k == 1 ? __builtin_fmaf(o[d], w0, sk[2 + d] * w) : __builtin_fmaf(sk[2 + d], w, o[d]);
             }
             const float inv = 1.0f / lt;
 #pragma unroll

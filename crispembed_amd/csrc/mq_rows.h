@@ -6,7 +6,7 @@ namespace mq {
 
 constexpr int ROWS_MAX_K = 4096;   // 16 blocks a wave
 constexpr int ROWS_MAX_LN = 1024;  // rows formed in registers, their quants in LDS
-constexpr int ROWS_MAX_T = 32;     // keys of one query, a lane each
+constexpr int ROWS_MAX_T = 32;     // keys of one query, a lane each; two blocks of the online softmax
 
 enum { ROWS_F32 = 0, ROWS_LN = 1, ROWS_Q = 2 };
 
@@ -35,8 +35,10 @@ struct RowsArgs {
 // with q_out (LayerNorm prologue only) instead gelu_erf of that, as the Q8_0 activation of the next
 // product (the GEMM workspace layout of M rows of n)
 hipError_t launch_rows(const void *image, int64_t n, int64_t k, RowsArgs a, void *q_out, hipStream_t s);
-// full attention over q|k|v rows of 3 H floats (bias added), T at most ROWS_MAX_T; the rows leave
-// as the Q8_0 activation of the o product in q_out
+// the same of quantized rows (a.x_ws) with the sums of the GEMM at 9 - 32 rows
+hipError_t launch_rows_groups(const void *image, int64_t n, int64_t k, RowsArgs a, hipStream_t s);
+// full attention over q|k|v rows of 3 H floats (bias added), T at most ROWS_MAX_T, head_dim 32 or 64;
+// the rows leave as the Q8_0 activation of the o product in q_out
 hipError_t launch_rows_attn(const float *qkv, void *q_out, int variant, int B, int T, int H, int nh, hipStream_t s);
 // true when the few-row form takes a Q8_0 encoder batch
 bool rows_path_fits(int64_t rows, int64_t T, int64_t H, int64_t F, int hd);

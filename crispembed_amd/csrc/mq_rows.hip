@@ -11,7 +11,11 @@
 // A LayerNorm needs whole rows, so the workgroups of a row tile (one per 32 output columns) each
 // form and quantize the tile's rows for themselves, while their weights are in flight; what a
 // workgroup can quantize for the next kernel (its 32 columns are one Q8_0 block of each row) it
-// does in its store.
+// does in its store.  Every value rounds as on the general path (mq_gemv.hip, mq_gemm.hip,
+// mq_encoder.hip, mq_quant.hip), whose results these layers give bit for bit: a quantized encoder
+// turns one other rounding of an activation, 1e-7, into 1e-3 of its output wherever that moves an
+// 8-bit value.
+#include <algorithm>
 #include <cstdlib>
 #include <type_traits>
 
@@ -40,6 +44,13 @@ __device__ __forceinline__ int rows_quant(float x, float id, int variant) {
     const float t = x * id;
     const float r = (variant == MQ_Q8_0_REF) ? roundf(t) : rintf(t);
     return (int)fminf(fmaxf(r, -128.f), 127.f);
+}
+
+// what a wave's lanes wrote to its own LDS is there for its other lanes
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // One value of 32 lanes (a half wave) as a Q8_0 block of row `row` and chunk kc of a GEMM-layout
@@ -115,7 +126,7 @@ __global__ __launch_bounds__(512) void k_rows(const RowsArgs a) {
     } else {
         const int nr = min((a.M - m0 - wave + 7) >> 3, 4);  // live rows of this wave
         if (nr > 0) {
-            float4 v[4][KP], res[PRO == ROWS_LN ? 4 : 1][KP], lw[KP], lb[KP];
+            float4 v[4][KP], res[4][KP], lw[KP], lb[KP];
 #pragma unroll
             for (int r = 0; r < 4; r++)
 #pragma unroll
@@ -137,48 +148,54 @@ __global__ __launch_bounds__(512) void k_rows(const RowsArgs a) {
                     if (c < a.K) lw[p] = *(const float4 *)(a.lw + c), lb[p] = *(const float4 *)(a.lb + c);
                 }
             weights();
+            if constexpr (PRO == ROWS_LN) {
+                // x + res here holds 4 values of a column step a lane, the statistics sum lane by
+                // lane over columns 64 apart (ln_stats): RB rows at a time change hands through LDS
+                constexpr int RB = KP <= 2 ? 4 : 2, V = 4 * KP;
+                float *xr = (float *)(smem + (size_t)nblk * (1024 + 128)) + wave * RB * a.K;
+#pragma unroll
+                for (int r0 = 0; r0 < 4; r0 += RB) {
+#pragma unroll
+                    for (int r = r0; r < r0 + RB; r++) {
+                        if (r >= nr) continue;  // uniform
+#pragma unroll
+                        for (int p = 0; p < KP; p++) {
+                            float4 &t = v[r][p];
+                            const float4 u = res[r][p];
+                            t.x = u.x + t.x, t.y = u.y + t.y, t.z = u.z + t.z, t.w = u.w + t.w;
+                            const int c = 256 * p + 4 * lane;
+                            if (c < a.K) *(float4 *)(xr + (r - r0) * a.K + c) = t;
+                        }
+                    }
+                    wave_lds_sync();
+#pragma unroll
+                    for (int r = r0; r < r0 + RB; r++) {
+                        if (r >= nr) continue;
+                        float t[V], mean, rstd;
+#pragma unroll
+                        for (int e = 0; e < V; e++) t[e] = lane + 64 * e < a.K ? xr[(r - r0) * a.K + lane + 64 * e] : 0.f;
+                        ln_stats(t, a.K, lane, a.eps, mean, rstd);
+#pragma unroll
+                        for (int p = 0; p < KP; p++) {
+                            float4 &x = v[r][p];
+                            x.x = ln_value(x.x, mean, rstd, lw[p].x, lb[p].x), x.y = ln_value(x.y, mean, rstd, lw[p].y, lb[p].y);
+                            x.z = ln_value(x.z, mean, rstd, lw[p].z, lb[p].z), x.w = ln_value(x.w, mean, rstd, lw[p].w, lb[p].w);
+                            const int c = 256 * p + 4 * lane;
+                            if (blockIdx.x == 0 && c < a.K)
+                                *(float4 *)(a.xout + (int64_t)(m0 + wave + 8 * r) * a.K + c) = x;
+                        }
+                    }
+                    wave_lds_sync();
+                }
+            }
             float am[4 * KP];
 #pragma unroll
-            for (int r = 0; r < 4; r++) {
-                if (PRO == ROWS_LN && r < nr) {  // uniform
-                    // the statistics in fp32 (their error scales a whole row, which its blocks' scales
-                    // take up), the values in fp64 up to the one rounding of the result
-                    float s = 0.f;
-#pragma unroll
-                    for (int p = 0; p < KP; p++) {
-                        const float4 t = v[r][p], u = res[PRO == ROWS_LN ? r : 0][p];
-                        s += ((t.x + u.x) + (t.y + u.y)) + ((t.z + u.z) + (t.w + u.w));
-                    }
-                    const float mean = wave_sum_f(s) / (float)a.K;
-                    float s2 = 0.f;
-#pragma unroll
-                    for (int p = 0; p < KP; p++)
-                        if (256 * p + 4 * lane < a.K) {
-                            const float4 t = v[r][p], u = res[PRO == ROWS_LN ? r : 0][p];
-                            const float x0 = (t.x + u.x) - mean, x1 = (t.y + u.y) - mean, x2 = (t.z + u.z) - mean,
-                                        x3 = (t.w + u.w) - mean;
-                            s2 += (x0 * x0 + x1 * x1) + (x2 * x2 + x3 * x3);
-                        }
-                    const double rstd = 1.0 / sqrt((double)wave_sum_f(s2) / (double)a.K + (double)a.eps);
-#pragma unroll
-                    for (int p = 0; p < KP; p++) {
-                        float4 &t = v[r][p];
-                        const float4 u = res[PRO == ROWS_LN ? r : 0][p];
-                        auto norm = [&](float x, float y, float w, float b) {
-                            return (float)(((double)x + (double)y - (double)mean) * rstd * (double)w + (double)b);
-                        };
-                        t.x = norm(t.x, u.x, lw[p].x, lb[p].x), t.y = norm(t.y, u.y, lw[p].y, lb[p].y);
-                        t.z = norm(t.z, u.z, lw[p].z, lb[p].z), t.w = norm(t.w, u.w, lw[p].w, lb[p].w);
-                        const int c = 256 * p + 4 * lane;
-                        if (blockIdx.x == 0 && c < a.K) *(float4 *)(a.xout + (int64_t)(m0 + wave + 8 * r) * a.K + c) = t;
-                    }
-                }
+            for (int r = 0; r < 4; r++)
 #pragma unroll
                 for (int p = 0; p < KP; p++) {
                     const float4 t = v[r][p];
                     am[4 * p + r] = max8(fmaxf(fmaxf(fabsf(t.x), fabsf(t.y)), fmaxf(fabsf(t.z), fabsf(t.w))));
                 }
-            }
             // the 8-lane groups hold one block each of every (r, p); lane g of a group divides for
             // block g of eight
             const int sub = lane & 7;
@@ -254,80 +271,178 @@ __global__ __launch_bounds__(512) void k_rows(const RowsArgs a) {
     }
 }
 
-// Attention of one (sequence, head) of at most ROWS_MAX_T tokens, fp32: q, k, v (bias added) to LDS, then
-// a wave per query row, lane j key j: score, softmax over the lanes, and lanes as head dims for
-// the weighted sum of V (64 / HD groups of keys side by side at HD < 64, HD / 64 dims a lane
-// above).  The rows leave as the Q8_0 activation of the o product (32 head dims a block).
-template <int HD>
+// The FFN-down product of 9 - 32 rows, which the general path gives to the GEMM: its sums, bit for bit
+// (the K-group form's: group g of four adds up blocks g, g + 4, ... in turn, the groups meet in
+// order, then the bias).  4 waves, wave g the group, over quantized rows; a round of PF blocks in
+// flight while the one before is summed.  What bounds it is its chain of K / 128 dependent steps and
+// the launch: 384 x 1536 at 16 rows 5.8 us (the GEMM 7.6; the eight-wave tree, other sums, 4.7).
+__global__ __launch_bounds__(256) void k_rows_groups(const RowsArgs a) {
+    constexpr int PF = 12;
+    __shared__ float part[4][16][64];
+    const int g = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+    const int l32 = lane & 31, half = lane >> 5;
+    const int n0 = blockIdx.x * 32, m0 = blockIdx.y * 32;
+    const int nblk = a.K >> 5;
+    struct Step {
+        v4i w, x;
+        float dw, dx;
+    } ra[PF], rb[PF];
+    auto load = [&](Step (&s)[PF], int kc0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < PF; i++) {
+            const int kc = min(kc0 + 4 * i, nblk - 1);
+            s[i].w = *(const v4i *)(a.wq + (((int64_t)blockIdx.x * a.kch + kc) << 10) + lane * 16);
+            s[i].x = *(const v4i *)(a.xq + (((int64_t)blockIdx.y * a.kch + kc) << 10) + lane * 16);
+            s[i].dw = a.wd[(int64_t)kc * a.n_pad + n0 + l32];
+            s[i].dx = a.xd[(int64_t)kc * a.m_pad + m0 + l32];
+        }
+    };
+    v16f acc = (v16f){};
+    auto compute = [&](const Step (&s)[PF], int kc0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < PF; i++)
+            if (kc0 + 4 * i < nblk) {  // uniform
+                const v16i I = __builtin_amdgcn_mfma_i32_32x32x32_i8(s[i].x, s[i].w, (v16i){}, 0, 0, 0);
+                const v16f P = __builtin_amdgcn_mfma_f32_32x32x2f32(half ? 0.f : s[i].dx, half ? 0.f : s[i].dw, (v16f){}, 0, 0, 0);
+#pragma unroll
+                for (int r = 0; r < 16; r++) acc[r] = __builtin_fmaf((float)I[r], P[r], acc[r]);
+            }
+    };
+    constexpr int D = 4 * PF;  // blocks a round
+    load(ra, g);
+    for (int kc0 = g; kc0 < nblk; kc0 += 2 * D) {
+        if (kc0 + D < nblk) load(rb, kc0 + D);
+        compute(ra, kc0);
+        if (kc0 + 2 * D < nblk) load(ra, kc0 + 2 * D);
+        if (kc0 + D < nblk) compute(rb, kc0 + D);
+    }
+#pragma unroll
+    for (int r = 0; r < 16; r++) part[g][r][lane] = acc[r];
+    const int col = n0 + l32;
+    const float bias = a.bias && col < a.N ? a.bias[col] : 0.f;
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+        const int r = 4 * g + u, row = m0 + 8 * g + 4 * half + u;
+        float s = ((part[0][r][lane] + part[1][r][lane]) + part[2][r][lane]) + part[3][r][lane];
+        if (a.bias) s += bias;
+        if (row < a.M && col < a.N) a.y[(int64_t)row * a.ldy + col] = s;
+    }
+}
+
+// Attention of one (sequence, head) of at most ROWS_MAX_T tokens: k_attention's values bit for bit
+// (its key ranges, key blocks and order of sums), with a wave per query row instead of a thread.
+// q (scaled), k, v (bias added) go to LDS; lane j takes key j: score, largest score so far of its key
+// range, probability; then lane d takes head dim d and sums the ranges side by side.  At HD 32
+// the two lane halves take half of the ranges each.  The rows leave as the Q8_0 activation of the
+// o product (32 head dims a block).
+template <int HD, int KS>
 __global__ __launch_bounds__(1024) void k_rows_attn(const float *__restrict__ qkv, int8_t *__restrict__ qo,
                                                     float *__restrict__ qd, int kch, int64_t m_pad, int variant, int T,
                                                     int H, int nh, float scale) {
     constexpr int ST = HD + 4;  // row stride: float4 reads of 8 consecutive rows hit all banks
-    constexpr int DL = HD < 64 ? 1 : HD / 64, KG = HD < 64 ? 64 / HD : 1;
+    constexpr int NG = HD == 32 && KS > 1 ? 2 : 1, NR = KS / NG;  // lane groups, ranges a lane
     extern __shared__ __attribute__((aligned(16))) float sm[];
     float *Q = sm, *K = Q + T * ST, *V = K + T * ST;
-    __shared__ float ps[16][64];
+    __shared__ float ps[16][ROWS_MAX_T], ms[16][4];  // scores, then probabilities; maxima of ranges or blocks
     const int b = blockIdx.x / nh, h = blockIdx.x % nh;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const float *base = qkv + (int64_t)b * T * 3 * H + h * HD;
     for (int e = threadIdx.x; e < 3 * T * (HD / 4); e += 1024) {
         const int d4 = e % (HD / 4), rest = e / (HD / 4), t = rest % T, w = rest / T;
-        *(float4 *)(Q + (w * T + t) * ST + 4 * d4) = *(const float4 *)(base + (int64_t)t * 3 * H + w * H + 4 * d4);
+        float4 x = *(const float4 *)(base + (int64_t)t * 3 * H + w * H + 4 * d4);
+        if (w == 0) x = make_float4(x.x * scale, x.y * scale, x.z * scale, x.w * scale);
+        *(float4 *)(Q + (w * T + t) * ST + 4 * d4) = x;
     }
     __syncthreads();
+    const int span = T / KS;                             // keys a range
+    const int jr = min(lane, T - 1) / span, j0 = jr * span;  // this lane's range and its first key
+    const int jb = (min(lane, T - 1) - j0) / ATT_KB;      // and its block in the range
+    const int d0 = lane % HD, g = NG > 1 ? lane / HD : 0;
     for (int i = wave; i < T; i += 16) {
-        float s = -INFINITY;
+        float s = 0.f;
         if (lane < T) {
-            float4 t = make_float4(0.f, 0.f, 0.f, 0.f), u = t;  // eight short chains
 #pragma unroll
-            for (int d = 0; d < HD; d += 8) {
-                const float4 q = *(const float4 *)(Q + i * ST + d), k = *(const float4 *)(K + lane * ST + d);
-                const float4 q2 = *(const float4 *)(Q + i * ST + d + 4), k2 = *(const float4 *)(K + lane * ST + d + 4);
-                t.x += q.x * k.x, t.y += q.y * k.y, t.z += q.z * k.z, t.w += q.w * k.w;
-                u.x += q2.x * k2.x, u.y += q2.y * k2.y, u.z += q2.z * k2.z, u.w += q2.w * k2.w;
+            for (int d4 = 0; d4 < HD / 4; d4++)
+                s = score4(s, *(const float4 *)(Q + i * ST + 4 * d4), *(const float4 *)(K + lane * ST + 4 * d4));
+            ps[wave][lane] = s;
+        }
+        wave_lds_sync();
+        float mx = -INFINITY;
+        const int j1 = min(j0 + ATT_KB * (jb + 1), j0 + span);
+        for (int c = j0; c < j1; c += 4)  // four reads in flight, the last key again past the end
+#pragma unroll
+            for (int u = 0; u < 4; u++) mx = fmaxf(mx, ps[wave][min(c + u, j1 - 1)]);
+        wave_lds_sync();
+        if (lane < T) {
+            ps[wave][lane] = expf(s - mx);
+            if (lane == j1 - 1) ms[wave][KS == 1 ? jb : jr] = mx;
+        }
+        wave_lds_sync();
+        float l[KS], o[KS], m[KS];
+#pragma unroll
+        for (int r = 0; r < NR; r++) {
+            const int k0 = (g * NR + r) * span;
+            l[r] = o[r] = 0.f;
+            m[r] = ms[wave][g * NR + r];
+            for (int c = 0; c < span; c += 4) {
+                if constexpr (KS == 1)  // one range of up to two blocks: the second rescales
+                    if (c == ATT_KB) {
+                        const float corr = expf(m[0] - ms[wave][1]);
+                        m[0] = ms[wave][1];
+                        l[0] *= corr, o[0] *= corr;
+                    }
+                float p[4], v[4];
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    const int j = k0 + min(c + u, span - 1);
+                    p[u] = ps[wave][j], v[u] = V[j * ST + d0];
+                }
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    const float ln = l[r] + p[u], on = __builtin_fmaf(p[u], v[u], o[r]);
+                    l[r] = c + u < span ? ln : l[r], o[r] = c + u < span ? on : o[r];
+                }
             }
-            s = (((t.x + t.y) + (t.z + t.w)) + ((u.x + u.y) + (u.z + u.w))) * scale;
         }
-        const float mx = wave_max_f(s);
-        const float p = lane < T ? expf(s - mx) : 0.f;
-        const float sum = wave_sum_f(p);
-        ps[wave][lane] = p;  // one wave writes and reads its row
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        const int d0 = lane % (HD < 64 ? HD : 64), g = KG > 1 ? lane / HD : 0;
-        float o[DL], o2[DL];
+        if constexpr (NG > 1)
 #pragma unroll
-        for (int n = 0; n < DL; n++) o[n] = o2[n] = 0.f;
-        int j = g;
-        for (; j + KG < T; j += 2 * KG) {
-            const float pj = ps[wave][j], pk = ps[wave][j + KG];
+            for (int r = 0; r < NR; r++) {
+                l[NR + r] = __shfl_xor(l[r], 32), o[NR + r] = __shfl_xor(o[r], 32), m[NR + r] = __shfl_xor(m[r], 32);
+            }
+        float lt = l[0], ot = o[0];
+        if constexpr (KS > 1) {  // lanes of the other half (g = 1) compute values that are not stored
+            float mt = m[0];
 #pragma unroll
-            for (int n = 0; n < DL; n++) {
-                o[n] += pj * V[j * ST + d0 + 64 * n];
-                o2[n] += pk * V[(j + KG) * ST + d0 + 64 * n];
+            for (int k = 1; k < KS; k++) mt = fmaxf(mt, m[k]);
+            const float w0 = expf(m[0] - mt);
+#pragma unroll
+            for (int k = 1; k < KS; k++) {
+                const float w = expf(m[k] - mt);
+                lt = k == 1 ? __builtin_fmaf(lt, w0, l[k] * w) : __builtin_fmaf(l[k], w, lt);
+                ot = k == 1 ? __builtin_fmaf(ot, w0, o[k] * w) : __builtin_fmaf(o[k], w, ot);
             }
         }
-        if (j < T) {
-            const float pj = ps[wave][j];
-#pragma unroll
-            for (int n = 0; n < DL; n++) o[n] += pj * V[j * ST + d0 + 64 * n];
-        }
-#pragma unroll
-        for (int n = 0; n < DL; n++) o[n] += o2[n];
-        if constexpr (KG > 1) o[0] += __shfl_xor(o[0], 32);
-#pragma unroll
-        for (int n = 0; n < DL; n++)
-            rows_store_q8_0(o[n] / sum, qo, qd, kch, m_pad, (int64_t)b * T + i, (h * HD + d0 + 64 * n) >> 5, lane & 31,
-                            variant, g == 0);
-        __builtin_amdgcn_wave_barrier();
+        const float inv = 1.0f / lt;
+        rows_store_q8_0(ot * inv, qo, qd, kch, m_pad, (int64_t)b * T + i, (h * HD + d0) >> 5, lane & 31, variant,
+                        lane < HD);
+        wave_lds_sync();
     }
 }
 
 template <int KP, int PRO, bool RQ = false>
 static hipError_t rows_cfg(const RowsArgs &a, hipStream_t s) {
-    const size_t op = PRO == ROWS_Q ? 0 : (size_t)(a.K / 32) * (1024 + 128), lds = op > 32768 ? op : 32768;
-    static_assert(ROWS_MAX_LN / 32 * (1024 + 128) <= 64 * 1024, "no raised LDS limit");
+    // fragments and row scales, the LayerNorm's rows of each wave; then the partial tiles
+    constexpr int RB = KP <= 2 ? 4 : 2;
+    const size_t op = (PRO == ROWS_Q ? 0 : (size_t)(a.K / 32) * (1024 + 128)) + (PRO == ROWS_LN ? (size_t)8 * RB * a.K * 4 : 0);
+    const size_t lds = op > 32768 ? op : 32768;
+    if constexpr (PRO == ROWS_LN) {
+        static std::atomic<bool> attr_set[MQ_MAX_DEVICES];
+        constexpr int most = KP * 8 * (1024 + 128) + 8 * RB * KP * 256 * 4;
+        static_assert(most <= 160 * 1024, "LDS budget");
+        const hipError_t e = dyn_lds_once((const void *)k_rows<KP, PRO, RQ>, most, attr_set);
+        if (e != hipSuccess) return e;
+    }
     hipLaunchKernelGGL((k_rows<KP, PRO, RQ>), dim3((unsigned)((a.N + 31) / 32), (unsigned)((a.M + 31) / 32)), dim3(512), lds,
                        s, a);
     return hipGetLastError();
@@ -370,47 +485,60 @@ hipError_t launch_rows(const void *image, int64_t n, int64_t k, RowsArgs a, void
     return k <= 512 ? rows_cfg<2, ROWS_F32>(a, s) : rows_cfg<4, ROWS_F32>(a, s);
 }
 
-hipError_t launch_rows_attn(const float *qkv, void *q_out, int variant, int B, int T, int H, int nh, hipStream_t s) {
-    const int hd = H / nh;
-    if (T <= 0 || T > ROWS_MAX_T || B <= 0 || (uintptr_t)qkv % 16) return hipErrorInvalidValue;
-    const ActPlanes o = act_planes(MQ_TYPE_Q8_0, (int64_t)B * T, H, true);
-    int8_t *qo = (int8_t *)q_out + o.xq;
-    float *qd = (float *)((char *)q_out + o.xd);
-    const int kch = (int)(o.kb_pad / 32);
-    const dim3 g((unsigned)(B * nh));
-    const size_t lds = (size_t)3 * T * (hd + 4) * sizeof(float);
-    const float scale = 1.0f / sqrtf((float)hd);
-    static_assert(3 * ROWS_MAX_T * (128 + 4) * 4 + 4096 <= 64 * 1024, "no raised LDS limit");
-    switch (hd) {
-        case 32:
-            hipLaunchKernelGGL((k_rows_attn<32>), g, dim3(1024), lds, s, qkv, qo, qd, kch, o.m_pad, variant, T, H, nh, scale);
-            break;
-        case 64:
-            hipLaunchKernelGGL((k_rows_attn<64>), g, dim3(1024), lds, s, qkv, qo, qd, kch, o.m_pad, variant, T, H, nh, scale);
-            break;
-        case 128:
-            hipLaunchKernelGGL((k_rows_attn<128>), g, dim3(1024), lds, s, qkv, qo, qd, kch, o.m_pad, variant, T, H, nh, scale);
-            break;
-        default: return hipErrorInvalidValue;
-    }
+hipError_t launch_rows_groups(const void *image, int64_t n, int64_t k, RowsArgs a, hipStream_t s) {
+    if (a.M <= 0) return hipSuccess;
+    if (k % 32 || !a.x_ws) return hipErrorInvalidValue;
+    const WeightPlanes p = weight_planes(MQ_TYPE_Q8_0, n, k);
+    const ActPlanes x = act_planes(MQ_TYPE_Q8_0, a.M, k, true);
+    a.wq = (const int8_t *)image + p.tq, a.wd = (const float *)((const char *)image + p.tdw);
+    a.xq = (const int8_t *)a.x_ws + x.xq, a.xd = (const float *)((const char *)a.x_ws + x.xd);
+    a.n_pad = (int)p.n_pad, a.m_pad = x.m_pad, a.kch = (int)(p.kb_pad / 32), a.N = (int)n, a.K = (int)k;
+    hipLaunchKernelGGL(k_rows_groups, dim3((unsigned)((a.N + 31) / 32), (unsigned)((a.M + 31) / 32)), dim3(256), 0, s, a);
     return hipGetLastError();
 }
 
-// Where the few-row form ends: its workgroups repeat a row tile's LayerNorm and quantization per 32
-// output columns, so it loses once a launch holds several of them per CU, sooner at wide rows; and
-// its attention walks T / 16 query rows a wave.  MI355X, microseconds a call, GEMM path (GEMV
-// path under 33 rows) / few rows, tokens B x T:
-//   H 384, F 1536, 6 layers:  1x16 489 / 175, 1x32 799 / 214, 2x32 240 / 219, 1x64 243 / 248,
-//                             4x32 243 / 222, 2x64 245 / 252, 16x16 277 / 270, 8x32 247 / 282
-//   H 768, F 3072, 3 layers:  1x16 324 / 138, 2x32 181 / 175, 1x64 181 / 191, 4x32 184 / 248
-//   H 1024, F 4096, 3 layers: 1x16 374 / 165, 2x32 214 / 204, 1x64 211 / 217, 4x32 216 / 283
-// MQ_BERT_ROWS sets the most rows it takes (0: none; measurements).
+template <int HD, int KS>
+static hipError_t rows_attn_cfg(const float *qkv, void *q_out, int variant, int B, int T, int H, int nh, hipStream_t s) {
+    const ActPlanes o = act_planes(MQ_TYPE_Q8_0, (int64_t)B * T, H, true);
+    const size_t lds = (size_t)3 * T * (HD + 4) * sizeof(float);
+    static_assert(3 * ROWS_MAX_T * (64 + 4) * 4 + 4096 <= 64 * 1024, "no raised LDS limit");
+    hipLaunchKernelGGL((k_rows_attn<HD, KS>), dim3((unsigned)(B * nh)), dim3(1024), lds, s, qkv, (int8_t *)q_out + o.xq,
+                       (float *)((char *)q_out + o.xd), (int)(o.kb_pad / 32), o.m_pad, variant, T, H, nh,
+                       1.0f / sqrtf((float)HD));
+    return hipGetLastError();
+}
+
+hipError_t launch_rows_attn(const float *qkv, void *q_out, int variant, int B, int T, int H, int nh, hipStream_t s) {
+    if (T <= 0 || T > ROWS_MAX_T || B <= 0 || (uintptr_t)qkv % 16) return hipErrorInvalidValue;
+    const int hd = H / nh, ks = T % 4 == 0 ? 4 : T % 2 == 0 ? 2 : 1;  // launch_attention's key ranges
+    static_assert(ROWS_MAX_T / 2 <= ATT_KB && ROWS_MAX_T <= 2 * ATT_KB, "one block a range, two in a single one");
+    switch (hd * 8 + ks) {
+        case 32 * 8 + 4: return rows_attn_cfg<32, 4>(qkv, q_out, variant, B, T, H, nh, s);
+        case 32 * 8 + 2: return rows_attn_cfg<32, 2>(qkv, q_out, variant, B, T, H, nh, s);
+        case 32 * 8 + 1: return rows_attn_cfg<32, 1>(qkv, q_out, variant, B, T, H, nh, s);
+        case 64 * 8 + 4: return rows_attn_cfg<64, 4>(qkv, q_out, variant, B, T, H, nh, s);
+        case 64 * 8 + 2: return rows_attn_cfg<64, 2>(qkv, q_out, variant, B, T, H, nh, s);
+        case 64 * 8 + 1: return rows_attn_cfg<64, 1>(qkv, q_out, variant, B, T, H, nh, s);
+        default: return hipErrorInvalidValue;
+    }
+}
+
+// The few-row form takes the batches whose products the general path gives to the GEMV (at most
+// GEMV_MAX_M rows) and whose attention is k_attention: those it computes bit for bit.  Up to 64 or 128
+// rows it would still be the faster one at some sizes (H 384, 6 layers: 2 x 32 tokens 247 -> 222 us,
+// 4 x 32 249 -> 225 us), but there the general path's sums are the GEMM's, and its attention the
+// matrix cores'.  MI355X, microseconds a call, general path / few rows, tokens B x T:
+//   H 384, F 1536, 6 layers:  1x5 302 / 152, 1x16 489 / 182, 1x32 804 / 225
+//   H 768, F 3072, 3 layers:  1x16 335 / 142
+//   H 1024, F 4096, 3 layers: 1x16 377 / 164
+// MQ_BERT_ROWS sets the most rows it takes (0: none; measurements, and comparing the two paths).
 bool rows_path_fits(int64_t rows, int64_t T, int64_t H, int64_t F, int hd) {
-    int64_t lim = H > 512 ? 64 : 128;
+    int64_t lim = GEMV_MAX_M;
     if (const char *e = getenv("MQ_BERT_ROWS"))
-        if (*e) lim = atoi(e);
+        if (*e) lim = std::min<int64_t>(lim, atoi(e));
+    auto gemv = [&](int64_t n, int64_t k) { return mq_mul_mat_path(MQ_TYPE_Q8_0, n, k, rows) == MQ_PATH_GEMV; };
     return rows <= lim && T <= ROWS_MAX_T && H <= ROWS_MAX_LN && F <= ROWS_MAX_K && H % 32 == 0 && F % 32 == 0 &&
-           (hd == 32 || hd == 64 || hd == 128);
+           (hd == 32 || hd == 64) && gemv(3 * H, H) && gemv(H, H) && gemv(F, H);
 }
 
 }  // namespace mq

@@ -99,3 +99,20 @@ def test_few_rows(oracle, H, nh, F, B, T, variant):
         _check(hp, O.Q8_0, B, T, f"rows_{H}_{F}", oracle)
     finally:
         mq.check(L.mq_set_q8_0_variant(saved))
+
+
+@pytest.mark.parametrize("H,nh,F,B,T", [
+    *[(96, 3, 544, 1, t) for t in range(1, 33)], *[(128, 2, 160, 1, t) for t in range(1, 33)],
+    (384, 12, 1536, 1, 16), (384, 12, 1536, 2, 4), (384, 6, 1536, 3, 3), (384, 12, 1536, 2, 16), (384, 12, 1536, 11, 3),
+    (512, 8, 2048, 4, 8), (768, 12, 3072, 2, 13), (1024, 16, 4096, 1, 31), (1024, 32, 4064, 5, 6), (992, 31, 32, 1, 9)])
+def test_few_rows_equal_the_general_path(H, nh, F, B, T, monkeypatch):
+    """The few-row layers change launches, not values: embeddings and hidden states are the bits of the
+    general path (MQ_BERT_ROWS=0), at every sequence length (the attention's key ranges and blocks
+    follow it), head_dim 32 and 64, row widths that are no multiple of 64 and of every step count,
+    under and over the 8 rows at which the FFN-down product's sums change, and just past 32 rows."""
+    hp = dict(SMALL)
+    hp.update(n_embd=H, n_head=nh, n_ff=F)
+    a = _run(hp, O.Q8_0, B, T, f"rows_eq_{H}_{nh}")
+    monkeypatch.setenv("MQ_BERT_ROWS", "0")
+    b = _run(hp, O.Q8_0, B, T, f"rows_eq_{H}_{nh}")
+    assert np.array_equal(a[3], b[3]) and np.array_equal(a[2], b[2])
