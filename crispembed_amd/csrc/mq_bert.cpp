@@ -133,6 +133,11 @@ extern "C" int mq_bert_encode(mq_bert *m, const int32_t *ids, const int32_t *typ
     const bool kquant = t == MQ_TYPE_Q4_K || t == MQ_TYPE_Q6_K;
     const bool ffn_fused = ((t == MQ_TYPE_Q8_0 && F % 128 == 0) || (kquant && gemm_requant_q8k_fits(t, rows, F))) &&
                            mq_mul_mat_path(t, F, H, rows) == MQ_PATH_GEMM && mq_mul_mat_path(t, H, F, rows) == MQ_PATH_GEMM;
+    // Q8_0 with every product on the GEMM path (below)
+    const int hd = (int)(H / hp.n_head);
+    const bool norm_fused = t == MQ_TYPE_Q8_0 && ffn_fused && H % 128 == 0 && H <= 1024 && (hd == 32 || hd == 64 || hd == 128) &&
+                            mq_mul_mat_path(t, 3 * H, H, rows) == MQ_PATH_GEMM &&
+                            mq_mul_mat_path(t, H, H, rows) == MQ_PATH_GEMM;
     const size_t wsb2 = ffn_fused ? mq_workspace_bytes(t, rows, F) : 0;
     if (!m->x.ensure(rows * H * f4) || !m->qkv.ensure(rows * 3 * H * f4) || !m->att.ensure(rows * H * f4) ||
         !m->y.ensure(rows * H * f4) || !m->ff.ensure(rows * F * f4) || !m->ws.ensure(wsb) ||
@@ -149,7 +154,7 @@ extern "C" int mq_bert_encode(mq_bert *m, const int32_t *ids, const int32_t *typ
         return rc;
     // a few rows of Q8_0: five launches a layer (mq_rows.hip) with the values of the loop below, bit for
     // bit; the products' biases added in their stores, the residual rows alternating between X and X2
-    if (t == MQ_TYPE_Q8_0 && rows_path_fits(rows, T, H, F, (int)(H / hp.n_head)) && (uintptr_t)X % 16 == 0) {
+    if (t == MQ_TYPE_Q8_0 && !norm_fused && rows_path_fits(rows, T, H, F, hd) && (uintptr_t)X % 16 == 0) {
         if (!m->x2.ensure(rows * H * f4) || !m->ws2.ensure(mq_workspace_bytes(t, rows, F)))
             return set_error(MQ_ENOMEM, "activation buffers for %lld rows", (long long)rows);
         float *X2 = m->x2.f();
@@ -190,10 +195,6 @@ extern "C" int mq_bert_encode(mq_bert *m, const int32_t *ids, const int32_t *typ
     // the GEMM stores, and the FFN intermediate never leaves the FFN-up GEMM (above).
     // Attention there is the fragment attention of FLASH_ATTN_EXT on strided views of the qkv
     // rows (the q/k/v biases added by the qkv GEMM's store).
-    const int hd = (int)(H / hp.n_head);
-    const bool norm_fused = t == MQ_TYPE_Q8_0 && ffn_fused && H % 128 == 0 && H <= 1024 && (hd == 32 || hd == 64 || hd == 128) &&
-                            mq_mul_mat_path(t, 3 * H, H, rows) == MQ_PATH_GEMM &&
-                            mq_mul_mat_path(t, H, H, rows) == MQ_PATH_GEMM;
     if (norm_fused) {
         auto strided = [&](float *p, int64_t ld) {  // [hd, T, n_head, B] over rows of ld floats
             mq_view v{};

@@ -333,15 +333,16 @@ __global__ __launch_bounds__(256) void k_rows_groups(const RowsArgs a) {
 // Attention of one (sequence, head) of at most ROWS_MAX_T tokens: k_attention's values bit for bit
 // (its key ranges, key blocks and order of sums), with a wave per query row instead of a thread.
 // q (scaled), k, v (bias added) go to LDS; lane j takes key j: score, largest score so far of its key
-// range, probability; then lane d takes head dim d and sums the ranges side by side.  At HD 32
-// the two lane halves take half of the ranges each.  The rows leave as the Q8_0 activation of the
-// o product (32 head dims a block).
+// range, probability; then lane d takes head dim d (and d + 64 at HD 128, which k_attention does
+// not have) and sums the ranges side by side.  At HD 32 the two lane halves take half of the ranges
+// each.  The rows leave as the Q8_0 activation of the o product (32 head dims a block).
 template <int HD, int KS>
 __global__ __launch_bounds__(1024) void k_rows_attn(const float *__restrict__ qkv, int8_t *__restrict__ qo,
                                                     float *__restrict__ qd, int kch, int64_t m_pad, int variant, int T,
                                                     int H, int nh, float scale) {
     constexpr int ST = HD + 4;  // row stride: float4 reads of 8 consecutive rows hit all banks
     constexpr int NG = HD == 32 && KS > 1 ? 2 : 1, NR = KS / NG;  // lane groups, ranges a lane
+    constexpr int DL = HD > 64 ? HD / 64 : 1;                            // dims a lane
     extern __shared__ __attribute__((aligned(16))) float sm[];
     float *Q = sm, *K = Q + T * ST, *V = K + T * ST;
     __shared__ float ps[16][ROWS_MAX_T], ms[16][4];  // scores, then probabilities; maxima of ranges or blocks
@@ -358,7 +359,7 @@ __global__ __launch_bounds__(1024) void k_rows_attn(const float *__restrict__ qk
     const int span = T / KS;                             // keys a range
     const int jr = min(lane, T - 1) / span, j0 = jr * span;  // this lane's range and its first key
     const int jb = (min(lane, T - 1) - j0) / ATT_KB;      // and its block in the range
-    const int d0 = lane % HD, g = NG > 1 ? lane / HD : 0;
+    const int d0 = lane % (HD < 64 ? HD : 64), g = NG > 1 ? lane / HD : 0;
     for (int i = wave; i < T; i += 16) {
         float s = 0.f;
         if (lane < T) {
@@ -379,38 +380,47 @@ __global__ __launch_bounds__(1024) void k_rows_attn(const float *__restrict__ qk
             if (lane == j1 - 1) ms[wave][KS == 1 ? jb : jr] = mx;
         }
         wave_lds_sync();
-        float l[KS], o[KS], m[KS];
+        float l[KS], o[KS][DL], m[KS];
 #pragma unroll
         for (int r = 0; r < NR; r++) {
             const int k0 = (g * NR + r) * span;
-            l[r] = o[r] = 0.f;
+            l[r] = 0.f;
+#pragma unroll
+            for (int n = 0; n < DL; n++) o[r][n] = 0.f;
             m[r] = ms[wave][g * NR + r];
             for (int c = 0; c < span; c += 4) {
                 if constexpr (KS == 1)  // one range of up to two blocks: the second rescales
                     if (c == ATT_KB) {
                         const float corr = expf(m[0] - ms[wave][1]);
                         m[0] = ms[wave][1];
-                        l[0] *= corr, o[0] *= corr;
+                        l[0] *= corr;
+#pragma unroll
+                        for (int n = 0; n < DL; n++) o[0][n] *= corr;
                     }
-                float p[4], v[4];
+                float p[4], v[4][DL];
 #pragma unroll
                 for (int u = 0; u < 4; u++) {
                     const int j = k0 + min(c + u, span - 1);
-                    p[u] = ps[wave][j], v[u] = V[j * ST + d0];
+                    p[u] = ps[wave][j];
+#pragma unroll
+                    for (int n = 0; n < DL; n++) v[u][n] = V[j * ST + d0 + 64 * n];
                 }
 #pragma unroll
                 for (int u = 0; u < 4; u++) {
-                    const float ln = l[r] + p[u], on = __builtin_fmaf(p[u], v[u], o[r]);
-                    l[r] = c + u < span ? ln : l[r], o[r] = c + u < span ? on : o[r];
+                    const bool in = c + u < span;
+                    l[r] = in ? l[r] + p[u] : l[r];
+#pragma unroll
+                    for (int n = 0; n < DL; n++) o[r][n] = in ? __builtin_fmaf(p[u], v[u][n], o[r][n]) : o[r][n];
                 }
             }
         }
         if constexpr (NG > 1)
 #pragma unroll
             for (int r = 0; r < NR; r++) {
-                l[NR + r] = __shfl_xor(l[r], 32), o[NR + r] = __shfl_xor(o[r], 32), m[NR + r] = __shfl_xor(m[r], 32);
+                l[NR + r] = __shfl_xor(l[r], 32), o[NR + r][0] = __shfl_xor(o[r][0], 32), m[NR + r] = __shfl_xor(m[r], 32);
             }
-        float lt = l[0], ot = o[0];
+        float lt = l[0];
+        float (&ot)[DL] = o[0];
         if constexpr (KS > 1) {  // lanes of the other half (g = 1) compute values that are not stored
             float mt = m[0];
 #pragma unroll
@@ -420,12 +430,16 @@ __global__ __launch_bounds__(1024) void k_rows_attn(const float *__restrict__ qk
             for (int k = 1; k < KS; k++) {
                 const float w = expf(m[k] - mt);
                 lt = k == 1 ? __builtin_fmaf(lt, w0, l[k] * w) : __builtin_fmaf(l[k], w, lt);
-                ot = k == 1 ? __builtin_fmaf(ot, w0, o[k] * w) : __builtin_fmaf(o[k], w, ot);
+#pragma unroll
+                for (int n = 0; n < DL; n++)
+                    ot[n] = k == 1 ? __builtin_fmaf(ot[n], w0, o[k][n] * w) : __builtin_fmaf(o[k][n], w, ot[n]);
             }
         }
         const float inv = 1.0f / lt;
-        rows_store_q8_0(ot * inv, qo, qd, kch, m_pad, (int64_t)b * T + i, (h * HD + d0) >> 5, lane & 31, variant,
-                        lane < HD);
+#pragma unroll
+        for (int n = 0; n < DL; n++)
+            rows_store_q8_0(ot[n] * inv, qo, qd, kch, m_pad, (int64_t)b * T + i, (h * HD + d0 + 64 * n) >> 5, lane & 31,
+                            variant, lane < HD);
         wave_lds_sync();
     }
 }
@@ -501,7 +515,7 @@ template <int HD, int KS>
 static hipError_t rows_attn_cfg(const float *qkv, void *q_out, int variant, int B, int T, int H, int nh, hipStream_t s) {
     const ActPlanes o = act_planes(MQ_TYPE_Q8_0, (int64_t)B * T, H, true);
     const size_t lds = (size_t)3 * T * (HD + 4) * sizeof(float);
-    static_assert(3 * ROWS_MAX_T * (64 + 4) * 4 + 4096 <= 64 * 1024, "no raised LDS limit");
+    static_assert(3 * ROWS_MAX_T * (128 + 4) * 4 + 4096 <= 64 * 1024, "no raised LDS limit");
     hipLaunchKernelGGL((k_rows_attn<HD, KS>), dim3((unsigned)(B * nh)), dim3(1024), lds, s, qkv, (int8_t *)q_out + o.xq,
                        (float *)((char *)q_out + o.xd), (int)(o.kb_pad / 32), o.m_pad, variant, T, H, nh,
                        1.0f / sqrtf((float)HD));
@@ -519,6 +533,9 @@ hipError_t launch_rows_attn(const float *qkv, void *q_out, int variant, int B, i
         case 64 * 8 + 4: return rows_attn_cfg<64, 4>(qkv, q_out, variant, B, T, H, nh, s);
         case 64 * 8 + 2: return rows_attn_cfg<64, 2>(qkv, q_out, variant, B, T, H, nh, s);
         case 64 * 8 + 1: return rows_attn_cfg<64, 1>(qkv, q_out, variant, B, T, H, nh, s);
+        case 128 * 8 + 4: return rows_attn_cfg<128, 4>(qkv, q_out, variant, B, T, H, nh, s);
+        case 128 * 8 + 2: return rows_attn_cfg<128, 2>(qkv, q_out, variant, B, T, H, nh, s);
+        case 128 * 8 + 1: return rows_attn_cfg<128, 1>(qkv, q_out, variant, B, T, H, nh, s);
         default: return hipErrorInvalidValue;
     }
 }
@@ -531,14 +548,16 @@ hipError_t launch_rows_attn(const float *qkv, void *q_out, int variant, int B, i
 //   H 384, F 1536, 6 layers:  1x5 302 / 152, 1x16 489 / 182, 1x32 804 / 225
 //   H 768, F 3072, 3 layers:  1x16 335 / 142
 //   H 1024, F 4096, 3 layers: 1x16 377 / 164
+// Head_dim 128, which k_attention does not take: up to 64 rows (128 at H <= 512), where the runner
+// has no other path (its fused GEMM path comes first).
 // MQ_BERT_ROWS sets the most rows it takes (0: none; measurements, and comparing the two paths).
 bool rows_path_fits(int64_t rows, int64_t T, int64_t H, int64_t F, int hd) {
-    int64_t lim = GEMV_MAX_M;
+    int64_t lim = hd < 128 ? GEMV_MAX_M : H > 512 ? 64 : 128;
     if (const char *e = getenv("MQ_BERT_ROWS"))
         if (*e) lim = std::min<int64_t>(lim, atoi(e));
     auto gemv = [&](int64_t n, int64_t k) { return mq_mul_mat_path(MQ_TYPE_Q8_0, n, k, rows) == MQ_PATH_GEMV; };
     return rows <= lim && T <= ROWS_MAX_T && H <= ROWS_MAX_LN && F <= ROWS_MAX_K && H % 32 == 0 && F % 32 == 0 &&
-           (hd == 32 || hd == 64) && gemv(3 * H, H) && gemv(H, H) && gemv(F, H);
+           (hd == 128 || ((hd == 32 || hd == 64) && gemv(3 * H, H) && gemv(H, H) && gemv(F, H)));
 }
 
 }  // namespace mq

@@ -83,12 +83,14 @@ def test_kv_direct_equals_kv_pass(monkeypatch):
 
 @pytest.mark.parametrize("H,nh,F,B,T", [
     (384, 12, 1536, 1, 1), (384, 12, 1536, 1, 31), (384, 12, 1536, 11, 3), (384, 12, 1536, 4, 32), (128, 4, 160, 3, 11),
-    (512, 8, 512, 4, 32), (768, 12, 3072, 2, 32), (1024, 8, 4096, 5, 7), (96, 3, 544, 1, 16)])
+    (512, 8, 512, 4, 32), (768, 12, 3072, 2, 32), (1024, 8, 4096, 5, 7), (96, 3, 544, 1, 16), (256, 2, 512, 1, 1),
+    (256, 2, 512, 1, 16), (1024, 8, 4096, 2, 14), (128, 1, 160, 3, 31)])
 @pytest.mark.parametrize("variant", [0, 2])
 def test_few_rows(oracle, H, nh, F, B, T, variant):
-    """The Q8_0 runner's few-row layers: edges of the 32-row tiles and of the 32-key attention,
-    head_dim 32 / 64 / 128, rows of every register width, widths that are no multiple of 128, two
-    rounding variants of the quantizer (0: x86; 2: reference), against the CPU encoder."""
+    """The Q8_0 runner at a few rows: the few-row layers up to 32 rows (head_dim 128: up to 128 where no
+    other path takes it), the GEMM path past them, edges of the 32-row tiles and of the 32-key
+    attention, rows of every register width, widths that are no multiple of 128, two rounding variants
+    of the quantizer (0: x86; 2: reference), against the CPU encoder."""
     from crispembed_amd import mq
     hp = dict(SMALL)
     hp.update(n_embd=H, n_head=nh, n_ff=F, n_max_pos=128)
