@@ -138,10 +138,13 @@ extern "C" int mq_bert_encode(mq_bert *m, const int32_t *ids, const int32_t *typ
     const bool norm_fused = t == MQ_TYPE_Q8_0 && ffn_fused && H % 128 == 0 && H <= 1024 && (hd == 32 || hd == 64 || hd == 128) &&
                             mq_mul_mat_path(t, 3 * H, H, rows) == MQ_PATH_GEMM &&
                             mq_mul_mat_path(t, H, H, rows) == MQ_PATH_GEMM;
-    const size_t wsb2 = ffn_fused ? mq_workspace_bytes(t, rows, F) : 0;
+    // the few-row layers' buffers too, for every batch they may get of up to this many rows: a handle
+    // that has seen its largest batch allocates nothing more (a later call may be under capture)
+    const int64_t few = t == MQ_TYPE_Q8_0 ? std::min(rows, rows_path_limit(H, F, hd)) : 0;
+    const size_t wsb2 = std::max(ffn_fused ? mq_workspace_bytes(t, rows, F) : 0, few ? mq_workspace_bytes(t, few, F) : 0);
     if (!m->x.ensure(rows * H * f4) || !m->qkv.ensure(rows * 3 * H * f4) || !m->att.ensure(rows * H * f4) ||
         !m->y.ensure(rows * H * f4) || !m->ff.ensure(rows * F * f4) || !m->ws.ensure(wsb) ||
-        (ffn_fused && !m->ws2.ensure(wsb2)))
+        !m->ws2.ensure(wsb2) || !m->x2.ensure(few * H * f4))
         return set_error(MQ_ENOMEM, "activation buffers for %lld rows", (long long)rows);
     hipStream_t s = (hipStream_t)stream;
     const float eps = hp.layer_norm_eps;
@@ -155,8 +158,6 @@ extern "C" int mq_bert_encode(mq_bert *m, const int32_t *ids, const int32_t *typ
     // a few rows of Q8_0: five launches a layer (mq_rows.hip) with the values of the loop below, bit for
     // bit; the products' biases added in their stores, the residual rows alternating between X and X2
     if (t == MQ_TYPE_Q8_0 && !norm_fused && rows_path_fits(rows, T, H, F, hd) && (uintptr_t)X % 16 == 0) {
-        if (!m->x2.ensure(rows * H * f4) || !m->ws2.ensure(mq_workspace_bytes(t, rows, F)))
-            return set_error(MQ_ENOMEM, "activation buffers for %lld rows", (long long)rows);
         float *X2 = m->x2.f();
         const int var = mq_q8_0_variant();
         // the product of layer_norm(y + res) (prev: the norm's parameters), of x, or of quantized rows

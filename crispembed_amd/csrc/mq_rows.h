@@ -40,7 +40,9 @@ hipError_t launch_rows_groups(const void *image, int64_t n, int64_t k, RowsArgs 
 // full attention over q|k|v rows of 3 H floats (bias added), T at most ROWS_MAX_T, head_dim 32, 64 or
 // 128; the rows leave as the Q8_0 activation of the o product in q_out
 hipError_t launch_rows_attn(const float *qkv, void *q_out, int variant, int B, int T, int H, int nh, hipStream_t s);
-// true when the few-row form takes a Q8_0 encoder batch
+// the most rows that the few-row form takes of a Q8_0 encoder's batches (0: none), and whether it takes
+// a batch
+int64_t rows_path_limit(int64_t H, int64_t F, int hd);
 bool rows_path_fits(int64_t rows, int64_t T, int64_t H, int64_t F, int hd);
 
 }  // namespace mq

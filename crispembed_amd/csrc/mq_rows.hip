@@ -551,13 +551,17 @@ hipError_t launch_rows_attn(const float *qkv, void *q_out, int variant, int B, i
 // Head_dim 128, which k_attention does not take: up to 64 rows (128 at H <= 512), where the runner
 // has no other path (its fused GEMM path comes first).
 // MQ_BERT_ROWS sets the most rows it takes (0: none; measurements, and comparing the two paths).
-bool rows_path_fits(int64_t rows, int64_t T, int64_t H, int64_t F, int hd) {
+int64_t rows_path_limit(int64_t H, int64_t F, int hd) {
+    if (H > ROWS_MAX_LN || F > ROWS_MAX_K || H % 32 || F % 32 || (hd != 32 && hd != 64 && hd != 128)) return 0;
     int64_t lim = hd < 128 ? GEMV_MAX_M : H > 512 ? 64 : 128;
     if (const char *e = getenv("MQ_BERT_ROWS"))
-        if (*e) lim = std::min<int64_t>(lim, atoi(e));
+        if (*e) lim = std::min<int64_t>(lim, std::max(atoi(e), 0));
+    return lim;
+}
+bool rows_path_fits(int64_t rows, int64_t T, int64_t H, int64_t F, int hd) {
     auto gemv = [&](int64_t n, int64_t k) { return mq_mul_mat_path(MQ_TYPE_Q8_0, n, k, rows) == MQ_PATH_GEMV; };
-    return rows <= lim && T <= ROWS_MAX_T && H <= ROWS_MAX_LN && F <= ROWS_MAX_K && H % 32 == 0 && F % 32 == 0 &&
-           (hd == 128 || ((hd == 32 || hd == 64) && gemv(3 * H, H) && gemv(H, H) && gemv(F, H)));
+    return rows <= rows_path_limit(H, F, hd) && T <= ROWS_MAX_T &&
+           (hd == 128 || (gemv(3 * H, H) && gemv(H, H) && gemv(F, H)));
 }
 
 }  // namespace mq

@@ -118,3 +118,42 @@ def test_few_rows_equal_the_general_path(H, nh, F, B, T, monkeypatch):
     monkeypatch.setenv("MQ_BERT_ROWS", "0")
     b = _run(hp, O.Q8_0, B, T, f"rows_eq_{H}_{nh}")
     assert np.array_equal(a[3], b[3]) and np.array_equal(a[2], b[2])
+
+
+@pytest.mark.parametrize("n_head,B,T", [(12, 1, 16), (12, 2, 16), (3, 1, 30)])
+def test_short_encode_captured_after_a_long_one(n_head, B, T):
+    """A handle that has encoded its largest batch allocates nothing for a shorter one, whatever layers
+    that takes: the short encode is captured (an allocation would break the capture) and every replay
+    gives the eager bits, with other work between the replays."""
+    import torch
+    from crispembed_amd import bert, synth
+    hp = dict(SMALL)
+    hp.update(n_embd=384, n_head=n_head, n_ff=1536)
+    enc = bert.BertEncoder(hp, O.Q8_0, bert.synthetic_weights(hp, O.Q8_0, name="cap"))
+    ids = torch.from_numpy(synth.integers("cap/ids", (8, 64), 400, 999).ravel().copy()).cuda()
+    big = torch.empty((8, 384), dtype=torch.float32, device="cuda")
+    out = torch.empty((B, 384), dtype=torch.float32, device="cuda")
+    hid = torch.empty((B * T, 384), dtype=torch.float32, device="cuda")
+    side = torch.cuda.Stream()
+
+    def encode(b, t, o, h=None):
+        enc.encode(ids.data_ptr(), b, t, o.data_ptr(), ctypes.c_void_p(side.cuda_stream),
+                   hidden_dev=h.data_ptr() if h is not None else None)
+
+    torch.cuda.synchronize()
+    encode(8, 64, big)
+    side.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        encode(B, T, out, hid)
+    torch.cuda.synchronize()
+    encode(B, T, out, hid)
+    side.synchronize()
+    ref = host(out).copy(), host(hid).copy()
+    for _ in range(3):
+        encode(8, 64, big)
+        side.synchronize()
+        out.fill_(float("nan")), hid.fill_(float("nan"))
+        torch.cuda.synchronize()
+        graph.replay()
+        assert np.array_equal(host(out), ref[0]) and np.array_equal(host(hid), ref[1])
