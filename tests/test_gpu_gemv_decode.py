@@ -245,6 +245,32 @@ def test_fused_gemv_silu_mul(gemv_form, wtype, m):
     del img
 
 
+@pytest.mark.parametrize("wtype", [O.Q4_K, O.Q6_K])
+@pytest.mark.parametrize("m", [1, 2, 8])
+def test_fused_gemv_nan_superblocks(gemv_form, wtype, m):
+    """ggml's quantizer compares |x| upwards from 0, so NaNs never set a superblock's scale: one of NaNs
+    only is a zero block, others quantize their numbers.  Every row count gives the quantizer's bits."""
+    import torch
+    from crispembed_amd import mq
+    n, k = 300, 6144
+    w = random_blocks(wtype, n, k, 11)
+    img = weight_image(wtype, w, n, k)
+    x = np.random.default_rng(m).standard_normal((m, k)).astype(np.float32)
+    x[0, :256] = np.nan                 # NaNs only
+    x[0, 2304:2560:3] = np.nan          # NaNs among numbers
+    x[m - 1, 4096:4352] = 0.0           # NaNs among zeros
+    x[m - 1, 4100:4200] = np.nan
+    x[m - 1, 6143] = np.nan
+    xd = dev(x)
+    got = _fused(wtype, [img], [n], k, xd, m)[0]
+    keep, wsp = _quant(wtype, xd, m, k)
+    ref = torch.full((m, n), np.nan, dtype=torch.float32, device="cuda")
+    mq.check(mq.lib().mq_mul_mat_q(wtype, ctypes.c_void_p(img[1]), n, k, ctypes.c_void_p(wsp), m,
+                                   ctypes.c_void_p(ref.data_ptr()), n, mq.PATH_GEMV, stream()))
+    assert np.isfinite(got).all() and np.array_equal(got.view(np.uint32), host(ref).view(np.uint32))
+    del img, keep
+
+
 def test_fused_gemv_lm_head(oracle, gemv_form, lm_head):
     """The Q6_K lm_head with the activation quantized inside the kernel, m = 1 and 8."""
     import torch
