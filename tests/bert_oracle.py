@@ -15,8 +15,8 @@ from ggml_numpy import q4_K_dequant, q6_K_dequant, q8_0_dequant, q8_K_fields
 _DEQ = {O.Q8_0: q8_0_dequant, O.Q4_K: q4_K_dequant, O.Q6_K: q6_K_dequant}
 
 
-def _act_deq(orc, wtype, x):
-    xq = orc.quantize_act(wtype, x)
+def _act_deq(orc, wtype, x, variant=O.Q8_0_X86):
+    xq = orc.quantize_act(wtype, x, variant)
     k = x.shape[1]
     if wtype == O.Q8_0:
         return q8_0_dequant(xq, k).astype(np.float64)
@@ -34,9 +34,9 @@ def _w_deq(wtype, w, k):
     return _DEQ[wtype](w, k).astype(np.float64)
 
 
-def linear(orc, wtype, x32, w, bias):
+def linear(orc, wtype, x32, w, bias, variant=O.Q8_0_X86):
     k = x32.shape[1]
-    y = (_act_deq(orc, wtype, x32) @ _w_deq(wtype, w, k).T).astype(np.float32)
+    y = (_act_deq(orc, wtype, x32, variant) @ _w_deq(wtype, w, k).T).astype(np.float32)
     return (y + bias).astype(np.float32)
 
 
@@ -53,8 +53,12 @@ def gelu_erf(x):
     return (0.5 * x * (1.0 + erf(x / np.sqrt(2.0)))).astype(np.float32)
 
 
-def encode(orc, hp, wtype, W, ids, types=None):
-    """ids (and token types, default 0) int32 [B, T] -> (pooled fp32 [B, H], last hidden fp32 [B*T, H])."""
+def encode(orc, hp, wtype, W, ids, types=None, variant=O.Q8_0_X86):
+    """ids (and token types, default 0) int32 [B, T] -> (pooled fp32 [B, H], last hidden fp32 [B*T, H]).
+    variant: the Q8_0 activation quantizer's rounding."""
+    def linear(orc, wtype, x, w, b):
+        return globals()["linear"](orc, wtype, x, w, b, variant)
+
     B, T = ids.shape
     H, nh = hp["n_embd"], hp["n_head"]
     hd = H // nh

@@ -30,7 +30,7 @@ def _both(L, mq, wtype, wp, n, k, x, path):
 
 
 @pytest.mark.parametrize("wtype", [O.Q8_0, O.Q4_K, O.Q6_K, O.F16])
-@pytest.mark.parametrize("path,m1,m2", [(2, 1000, 300), (1, 8, 3), (0, 4096, 5)])
+@pytest.mark.parametrize("path,m1,m2", [(2, 1000, 300), (1, 8, 3), (0, 4096, 5), (0, 32, 9)])
 def test_noalloc_equals_mul_mat_ex(oracle, wtype, path, m1, m2):
     from crispembed_amd import mq
     L = mq.lib()
