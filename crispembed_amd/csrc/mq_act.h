@@ -28,6 +28,22 @@ __device__ __forceinline__ float silu_mul_f32(float g, float u) {
     return (g / (1.0f + expf(-g))) * u;
 }
 
+// ggml's Q8_0 scale of a block whose largest magnitude is amax (d, as stored: rounded through fp16)
+// and its reciprocal, and one quant (variant: quantize_row_q8_0 of MQ_Q8_0_*)
+__device__ __forceinline__ void q8_0_scale(float amax, int variant, float &d, float &id) {
+#pragma clang fp contract(off)
+    const float dd = amax / 127.f;
+    if (variant == MQ_Q8_0_X86) id = (amax != 0.0f) ? 127.f / amax : 0.0f;
+    else id = (dd != 0.0f) ? 1.0f / dd : 0.0f;
+    d = f16_bits_to_f32(f32_to_f16_bits(dd));
+}
+__device__ __forceinline__ int q8_0_quant(float x, float id, int variant) {
+#pragma clang fp contract(off)
+    const float t = x * id;
+    const float r = (variant == MQ_Q8_0_REF) ? roundf(t) : rintf(t);
+    return (int)fminf(fmaxf(r, -128.f), 127.f);
+}
+
 // Half of one Q8_0 block of a kernel's quantized output: this lane's 16 values, the other 16
 // in lane l ^ 32.  The values are op(v) (pre: MQ_PRE_NONE or MQ_PRE_GELU_ERF; rows that are
 // not live: zero, as the activation quantizer's pad rows), and the block is quantized as
@@ -46,25 +62,18 @@ __device__ __forceinline__ float requant_q8_0(float (&v)[16], bool live, int pre
 #pragma unroll
     for (int e = 1; e < 16; e++) amax = fmaxf(amax, fabsf(v[e]));
     amax = fmaxf(amax, __shfl_xor(amax, 32));
-    const float d = amax / 127.f;
-    float id;
-    if (variant == MQ_Q8_0_X86) id = (amax != 0.0f) ? 127.f / amax : 0.0f;
-    else id = (d != 0.0f) ? 1.0f / d : 0.0f;
+    float d, id;
+    q8_0_scale(amax, variant, d, id);
     uint32_t w[4];
 #pragma unroll
     for (int u = 0; u < 4; u++) {
         uint32_t pk = 0;
 #pragma unroll
-        for (int b = 0; b < 4; b++) {
-            const float t = v[4 * u + b] * id;
-            float r = (variant == MQ_Q8_0_REF) ? roundf(t) : rintf(t);
-            r = fminf(fmaxf(r, -128.f), 127.f);
-            pk |= ((uint32_t)((int)r & 0xff)) << (8 * b);
-        }
+        for (int b = 0; b < 4; b++) pk |= ((uint32_t)(q8_0_quant(v[4 * u + b], id, variant) & 0xff)) << (8 * b);
         w[u] = pk;
     }
     q = make_uint4(w[0], w[1], w[2], w[3]);
-    return f16_bits_to_f32(f32_to_f16_bits(d));
+    return d;
 }
 
 

@@ -305,6 +305,7 @@ __device__ __forceinline__ void gv_quantize_sb(const GvX &X, int sb, int M, int 
                                                _Float16 *gs) {
 #pragma clang fp contract(off)
     constexpr int LPR = QK_K / VPL, RPP = 64 / LPR;  // lanes per row, rows per pass
+    static_assert(LPR < 64, "one row takes gv_quantize_row");
     const int r0 = lane / LPR, p = lane % LPR, gbase = lane - p;
     for (int rb = 0; rb < M; rb += RPP) {
         const int m = rb + r0;
@@ -339,7 +340,7 @@ __device__ __forceinline__ void gv_quantize_sb(const GvX &X, int sb, int M, int 
 #pragma unroll
         for (int off = LPR / 2; off >= 1; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, LPR));
         const unsigned long long hit = __ballot(la == amax) >> gbase;
-        const unsigned long long row_hits = LPR == 64 ? hit : (hit & ((1ull << LPR) - 1));
+        const unsigned long long row_hits = hit & ((1ull << LPR) - 1);
         const float mx = __shfl(lm, gbase + __ffsll((long long)row_hits) - 1);
         uint32_t w[VPL / 4];
 #pragma unroll
@@ -379,8 +380,8 @@ __device__ __forceinline__ void gv_quantize_sb(const GvX &X, int sb, int M, int 
 // before the first is used, the reductions interleave and share the divisions, and the bytes are
 // gv_quantize_sb's.  A decode step is a chain of such kernels, so their latency is its time: with the
 // superblocks one after the other the Q4_K 2048 x 6144 product on silu(gate) up took 9.4 us a
-// launch and a step of 28 layers 708 us, side by side 666 us (MI355X).  At M >= 2 the four-rows-at-once
-// form of gv_quantize_sb is the faster one (a step at M = 2 - 8: 623 against 714 us).
+// launch and a step of 28 layers (2048 / 6144, four launches each) 708 us, side by side 664 us (MI355X).
+// M = 2 takes gv_quantize_sb two rows at a time, M > 2 four.
 template <int NS>
 __device__ __forceinline__ void gv_quantize_row(const GvX &X, int sb0, int nsb, int lane, int8_t (*qs)[GEMV_CHUNK * QK_K],
                                                 float (*ds)[GEMV_CHUNK], _Float16 (*gs)[GEMV_CHUNK * 16]) {

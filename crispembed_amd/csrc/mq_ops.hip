@@ -286,21 +286,14 @@ __global__ __launch_bounds__(64 * NW) void k_norm_q8_0(const float *x, const flo
             amax = fmaxf(amax, __shfl_xor(amax, 1));
             amax = fmaxf(amax, __shfl_xor(amax, 2));
             amax = fmaxf(amax, __shfl_xor(amax, 4));
-            const float dq = amax / 127.f;
-            float id;
-            if (variant == MQ_Q8_0_X86) id = (amax != 0.0f) ? 127.f / amax : 0.0f;
-            else id = (dq != 0.0f) ? 1.0f / dq : 0.0f;
+            float dq, id;
+            q8_0_scale(amax, variant, dq, id);
             uint32_t pk = 0;
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const float t = y[e] * id;
-                float q = (variant == MQ_Q8_0_REF) ? roundf(t) : rintf(t);
-                q = fminf(fmaxf(q, -128.f), 127.f);
-                pk |= ((uint32_t)((int)q & 0xff)) << (8 * e);
-            }
+            for (int e = 0; e < 4; e++) pk |= ((uint32_t)(q8_0_quant(y[e], id, variant) & 0xff)) << (8 * e);
             const int c = 4 * p + (sub >> 3), cbyte = 4 * (sub & 7);  // chunk, byte within it
             *(uint32_t *)(frag + c * FST + ((rr + 32 * (cbyte >> 4)) << 4) + (cbyte & 15)) = pk;
-            if ((sub & 7) == 0) dsh[c][rr] = f16_bits_to_f32(f32_to_f16_bits(dq));
+            if ((sub & 7) == 0) dsh[c][rr] = dq;
         }
     }
     __syncthreads();

@@ -80,27 +80,19 @@ __global__ __launch_bounds__(256) void k_quantize_q8_0(const float *__restrict__
     amax = fmaxf(amax, __shfl_xor(amax, 1, 8));
     amax = fmaxf(amax, __shfl_xor(amax, 2, 8));
     amax = fmaxf(amax, __shfl_xor(amax, 4, 8));
-    const float d = amax / 127.f;
-    float id;
-    if (VARIANT == MQ_Q8_0_X86) id = (amax != 0.0f) ? 127.f / amax : 0.0f;
-    else id = (d != 0.0f) ? 1.0f / d : 0.0f;
-    auto q = [&](float xv) -> uint32_t {
-        const float t = xv * id;
-        float r = (VARIANT == MQ_Q8_0_REF) ? roundf(t) : rintf(t);
-        r = fminf(fmaxf(r, -128.f), 127.f);
-        return (uint32_t)((int)r & 0xff);
-    };
+    float d, id;
+    q8_0_scale(amax, VARIANT, d, id);
+    auto q = [&](float xv) -> uint32_t { return (uint32_t)(q8_0_quant(xv, id, VARIANT) & 0xff); };
     const uint32_t packed = q(v.x) | (q(v.y) << 8) | (q(v.z) << 16) | (q(v.w) << 24);
-    const uint16_t dh = f32_to_f16_bits(d);
     if (OUT == OUT_ROWS) {
         *(uint32_t *)(out + row * k + b * QK8_0 + sub * 4) = packed;
-        if (sub == 0) xd[row * nbr + b] = f16_bits_to_f32(dh);
+        if (sub == 0) xd[row * nbr + b] = d;
     } else {
         uint8_t *blkp = (uint8_t *)out + (row * nbr + b) * sizeof(block_q8_0);
         uint16_t *qs16 = (uint16_t *)(blkp + 2 + sub * 4);  // 2-byte aligned in the 34-byte block
         qs16[0] = (uint16_t)(packed & 0xffff);
         qs16[1] = (uint16_t)(packed >> 16);
-        if (sub == 0) *(uint16_t *)blkp = dh;
+        if (sub == 0) *(uint16_t *)blkp = f32_to_f16_bits(d);  // exact
     }
 }
 
@@ -296,18 +288,11 @@ __global__ __launch_bounds__(256) void k_quantize_tiled(const float *__restrict_
             *(uint2 *)dst = o;
         } else if constexpr (FMT == TQ_Q8_0) {
             const float amax = max8(fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
-            const float d = amax / 127.f;
-            float id;
-            if (VARIANT == MQ_Q8_0_X86) id = (amax != 0.0f) ? 127.f / amax : 0.0f;
-            else id = (d != 0.0f) ? 1.0f / d : 0.0f;
-            auto q = [&](float xv) -> uint32_t {
-                const float t = xv * id;
-                float rr = (VARIANT == MQ_Q8_0_REF) ? roundf(t) : rintf(t);
-                rr = fminf(fmaxf(rr, -128.f), 127.f);
-                return (uint32_t)((int)rr & 0xff);
-            };
+            float d, id;
+            q8_0_scale(amax, VARIANT, d, id);
+            auto q = [&](float xv) -> uint32_t { return (uint32_t)(q8_0_quant(xv, id, VARIANT) & 0xff); };
             *(uint32_t *)dst = q(v.x) | (q(v.y) << 8) | (q(v.z) << 16) | (q(v.w) << 24);
-            if ((sub & 7) == 0) dsh[c][r] = f16_bits_to_f32(f32_to_f16_bits(d));
+            if ((sub & 7) == 0) dsh[c][r] = d;
         }
     }
     __syncthreads();

@@ -31,21 +31,6 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 
-// ggml's Q8_0 scale and reciprocal of a block whose largest magnitude is amax, and one quant
-__device__ __forceinline__ void rows_scale(float amax, int variant, float &d, float &id) {
-#pragma clang fp contract(off)
-    const float dd = amax / 127.f;
-    if (variant == MQ_Q8_0_X86) id = (amax != 0.0f) ? 127.f / amax : 0.0f;
-    else id = (dd != 0.0f) ? 1.0f / dd : 0.0f;
-    d = f16_bits_to_f32(f32_to_f16_bits(dd));
-}
-__device__ __forceinline__ int rows_quant(float x, float id, int variant) {
-#pragma clang fp contract(off)
-    const float t = x * id;
-    const float r = (variant == MQ_Q8_0_REF) ? roundf(t) : rintf(t);
-    return (int)fminf(fmaxf(r, -128.f), 127.f);
-}
-
 // what a wave's lanes wrote to its own LDS is there for its other lanes
 __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -61,20 +46,14 @@ __device__ __forceinline__ void rows_store_q8_0(float x, int8_t *qo, float *qd, 
     amax = fmaxf(amax, dpp_f<0x140>(amax));
     amax = fmaxf(amax, __shfl_xor(amax, 16));
     float d, id;
-    rows_scale(amax, variant, d, id);
+    q8_0_scale(amax, variant, d, id);
     if (live) {
         qo[(((row >> 5) * kch + kc) << 10) + ((((l32 >> 4) << 5) + (row & 31)) << 4) + (l32 & 15)] =
-            (int8_t)rows_quant(x, id, variant);
+            (int8_t)q8_0_quant(x, id, variant);
         if (l32 == 0) qd[kc * m_pad + row] = d;
     }
 }
 
-// The few-row product.  8 waves; wave w multiplies the 32-value blocks w, w + 8, ... of K (one
-// v_mfma_i32_32x32x32_i8 and a scaled add each), and the eight partial tiles meet in LDS.  The sums
-// are the GEMV's, in its order, so the results are its results bit for bit: there lane l of a wave
-// adds up blocks l and l + 64 and the lanes meet in a tree over lane ^ 32, 16, 8, 4, 2, 1; here block
-// l = w + 8 i is step i of wave w, so the tree's first three levels join steps i ^ 4, 2, 1 of a wave
-// and the last three join waves w ^ 4, 2, 1.
 // rows_tree<KP, I, S>: the sum of steps I, I + S, I + 2 S, ... < min(KP, 8), as the GEMV's lanes meet
 // (a step that is not there is +0 in the GEMV, and no step's sum is -0: it drops out)
 template <int KP, int I, int S, class F>
@@ -88,6 +67,12 @@ __device__ __forceinline__ v16f rows_tree(F &&leaf) {
     }
 }
 
+// The few-row product.  8 waves; wave w multiplies the 32-value blocks w, w + 8, ... of K (one
+// v_mfma_i32_32x32x32_i8 and a scaled add each), and the eight partial tiles meet in LDS.  The sums
+// are the GEMV's, in its order, so the results are its results bit for bit: there lane l of a wave
+// adds up blocks l and l + 64 and the lanes meet in a tree over lane ^ 32, 16, 8, 4, 2, 1; here block
+// l = w + 8 i is step i of wave w, so the tree's first three levels join steps i ^ 4, 2, 1 of a wave
+// and the last three join waves w ^ 4, 2, 1.
 // PRO: the rows.  ROWS_Q: quantized already (GEMM layout), fragments straight to registers.
 // ROWS_F32, ROWS_LN: wave w forms rows w, w + 8, w + 16, w + 24 (lane l values 256 p + 4 l .. + 3, p < KP =
 // ceil(K / 256)), as they are or as layer_norm(x + res), quantizes them and leaves them in LDS
@@ -205,7 +190,7 @@ __global__ __launch_bounds__(512) void k_rows(const RowsArgs a) {
 #pragma unroll
                 for (int g = 1; g < 8; g++) mine = sub == g ? am[g0 + g] : mine;
                 float d, id;
-                rows_scale(mine, a.variant, d, id);
+                q8_0_scale(mine, a.variant, d, id);
                 const int pd = (g0 + sub) >> 2, kd = 8 * pd + (lane >> 3);
                 if (kd < nblk) sd[kd * 32 + wave + 8 * (sub & 3)] = d;
 #pragma unroll
@@ -214,8 +199,8 @@ __global__ __launch_bounds__(512) void k_rows(const RowsArgs a) {
                     if (r >= nr) continue;  // uniform
                     const float ig = __shfl(id, (lane & 56) + g);
                     const float4 t = v[r][p];
-                    const uint32_t q = pack4_i8(rows_quant(t.x, ig, a.variant), rows_quant(t.y, ig, a.variant),
-                                                rows_quant(t.z, ig, a.variant), rows_quant(t.w, ig, a.variant));
+                    const uint32_t q = pack4_i8(q8_0_quant(t.x, ig, a.variant), q8_0_quant(t.y, ig, a.variant),
+                                                q8_0_quant(t.z, ig, a.variant), q8_0_quant(t.w, ig, a.variant));
                     if (kc < nblk)
                         *(uint32_t *)(frag + (kc << 10) + (((w0 >> 4) << 5) + wave + 8 * r) * 16 + (w0 & 15)) = q;
                 }
