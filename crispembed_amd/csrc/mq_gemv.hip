@@ -404,12 +404,12 @@ __device__ __forceinline__ void gv_quantize_row(const GvX &X, int sb0, int nsb, 
     uint32_t q[NS];
     int bs[NS];
     float d[NS];
-    q8_K_rows<NS>(v, lane, q, bs, d);
+    q8_K_rows<NS, true>(v, lane, q, bs, d);
 #pragma unroll
     for (int i = 0; i < NS; i++) {
         if (sb0 + 8 * i >= nsb) continue;  // uniform
         *(uint32_t *)(qs[i] + 4 * lane) = q[i];
-        if (lane == 0) ds[i][0] = d[i] == d[i] ? d[i] : 0.f;  // a superblock of NaNs only: a zero block
+        if (lane == 0) ds[i][0] = d[i];
         if ((lane & 7) == 0) {
             gs[i][lane >> 3] = (_Float16)(bs[i] & 63);
             gs[i][8 + (lane >> 3)] = (_Float16)((bs[i] >> 6) * 64);

@@ -101,8 +101,9 @@ __device__ __forceinline__ void q8_K_block_row(const float4 v, int lane, int r, 
 // of sub-block j's 32 quants) in lane 8j of bs[i], the scale 1 / iscale in d[i] (wave-uniform).
 // The NR scales' two divisions (-127 / max and 1 / iscale, wave-uniform values) run once for all
 // rows -- row i's operand in lane i -- instead of once per row, which was a quarter of the row's
-// instructions.  Bit for bit q8_K_block_row's results.
-template <int NR>
+// instructions.  Bit for bit q8_K_block_row's results.  NAN_ZERO: a block of NaNs only is a zero block,
+// as in quantize_row_q8_K, whose comparisons start at 0 (else its scale is NaN).
+template <int NR, bool NAN_ZERO = false>
 __device__ __forceinline__ void q8_K_rows(const float4 *v, int lane, uint32_t *q, int *bs, float *d) {
 #pragma clang fp contract(off)
     static_assert(NR >= 1 && NR <= 64, "rows per wave");
@@ -114,7 +115,7 @@ __device__ __forceinline__ void q8_K_rows(const float4 *v, int lane, uint32_t *q
         first_absmax4(vals, la, lm);
         amax[i] = wave_max_f(la);
         const unsigned long long hit = __ballot(la == amax[i]);
-        mx[i] = amax[i] != 0.0f ? lane_f(lm, __ffsll((long long)hit) - 1) : 1.0f;
+        mx[i] = (NAN_ZERO ? amax[i] > 0.0f : amax[i] != 0.0f) ? lane_f(lm, __ffsll((long long)hit) - 1) : 1.0f;
     }
     float m = 1.0f;
 #pragma unroll
@@ -126,7 +127,7 @@ __device__ __forceinline__ void q8_K_rows(const float4 *v, int lane, uint32_t *q
         uint32_t packed = 0;
         int s16 = 0;
         float dval = 0.0f;
-        if (amax[i] != 0.0f) {
+        if (NAN_ZERO ? amax[i] > 0.0f : amax[i] != 0.0f) {
             const float iscale = lane_f(is_l, i);
             int qv[4];
 #pragma unroll
