@@ -114,9 +114,9 @@ def test_attention_sink(causal, hd, nq, nkv, g, form, monkeypatch):
 @pytest.mark.parametrize("hd,nq,nkv", [(64, 2, 2), (128, 4, 2), (128, 3, 1)])
 def test_attention_climbing_scores(causal, hd, nq, nkv, climb, form, monkeypatch):
     """Scores that climb (or fall) by `climb` powers of two from one 32-key block to the next: the
-    online softmax moves its exponent only past 8, so 5 takes it every second block, 12 every
-    block, -12 never.  Bound: a score's operands are split to 2^-22 each, so at |s| <= 7 blocks x
-    12 ln 2 = 58 a probability is off by 58 x 2^-21 = 2.8e-5 at most."""
+    online softmax rescales what it has at every block on the way up, and never on the way down.
+    Bound: a score's operands are split to 2^-22 each, so at |s| <= 7 blocks x 12 ln 2 = 58 a
+    probability is off by 58 x 2^-21 = 2.8e-5 at most."""
     from crispembed_amd import mq
     import torch
     if form == "frag":
