@@ -56,8 +56,8 @@ def gelu_erf(x):
 def encode(orc, hp, wtype, W, ids, types=None, variant=O.Q8_0_X86):
     """ids (and token types, default 0) int32 [B, T] -> (pooled fp32 [B, H], last hidden fp32 [B*T, H]).
     variant: the Q8_0 activation quantizer's rounding."""
-    def linear(orc, wtype, x, w, b):
-        return globals()["linear"](orc, wtype, x, w, b, variant)
+    def lin(x32, w, bias):
+        return linear(orc, wtype, x32, w, bias, variant)
 
     B, T = ids.shape
     H, nh = hp["n_embd"], hp["n_head"]
@@ -67,17 +67,17 @@ def encode(orc, hp, wtype, W, ids, types=None, variant=O.Q8_0_X86):
     x = (x + (W["type"][0] if types is None else W["type"][np.asarray(types).ravel()])).astype(np.float32)
     x = layernorm(x, W["ln_w"], W["ln_b"], eps)
     for lay in W["layers"]:
-        q = linear(orc, wtype, x, lay["wq"], lay["bq"]).astype(np.float64).reshape(B, T, nh, hd)
-        k = linear(orc, wtype, x, lay["wk"], lay["bk"]).astype(np.float64).reshape(B, T, nh, hd)
-        v = linear(orc, wtype, x, lay["wv"], lay["bv"]).astype(np.float64).reshape(B, T, nh, hd)
+        q = lin(x, lay["wq"], lay["bq"]).astype(np.float64).reshape(B, T, nh, hd)
+        k = lin(x, lay["wk"], lay["bk"]).astype(np.float64).reshape(B, T, nh, hd)
+        v = lin(x, lay["wv"], lay["bv"]).astype(np.float64).reshape(B, T, nh, hd)
         s = np.einsum("bihd,bjhd->bhij", q, k) / np.sqrt(hd)
         s = np.exp(s - s.max(-1, keepdims=True))
         p = s / s.sum(-1, keepdims=True)
         a = np.einsum("bhij,bjhd->bihd", p, v).reshape(B * T, H).astype(np.float32)
-        o = linear(orc, wtype, a, lay["wo"], lay["bo"])
+        o = lin(a, lay["wo"], lay["bo"])
         x = layernorm(x.astype(np.float64) + o, lay["ln1_w"], lay["ln1_b"], eps)
-        h = gelu_erf(linear(orc, wtype, x, lay["wfc1"], lay["bfc1"]))
-        f = linear(orc, wtype, h, lay["wfc2"], lay["bfc2"])
+        h = gelu_erf(lin(x, lay["wfc1"], lay["bfc1"]))
+        f = lin(h, lay["wfc2"], lay["bfc2"])
         x = layernorm(x.astype(np.float64) + f, lay["ln2_w"], lay["ln2_b"], eps)
     pooled = x.astype(np.float64).reshape(B, T, H).mean(1)
     norm = np.sqrt(np.maximum((pooled ** 2).sum(-1, keepdims=True), 1e-12))
